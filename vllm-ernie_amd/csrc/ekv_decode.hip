@@ -749,30 +749,41 @@ sparse_decode_kernel(DecodeArgs a) {
   }
 }
 
-// 256 threads per (t, 4 heads): wave = head, lane = 8 output channels.  Rows
-// finished by their only split are skipped.
+// Merges a row's splits: kW waves per (t, head), lane = 8 output channels.
+// Wave w of a head sums splits w, w + kW, ...; with kW = 4 the four sums meet
+// in LDS, each thread finishing two channels.  Bound by memory latency (the
+// partials, 2 KB per split and head, come from other XCDs' writes), so the
+// splits' loads go out together.  Many splits a row: 4 waves (one row of 68
+// splits: 6.7 us, 14.7 with a wave per head); few: a wave per head (32 rows of
+// 8: 8.4 us, 10.4 with 4 waves; 64 of 4: 7.6, 12.7).  Rows finished by their
+// only split are skipped.
+template <int kW>
 __global__ void __launch_bounds__(256) decode_combine_kernel(
     const float* ws_o, const float* ws_ml, const int2* ws_rows, int32_t heads, const float* sinks,
     uint16_t* out, int64_t out_tok_stride, int64_t out_head_stride, float* lse, int64_t lse_stride) {
-  const int t = blockIdx.y;
-  const int h = 4 * blockIdx.x + (threadIdx.x >> 6);
+  __shared__ __align__(16) float s_acc[kW > 1 ? kW : 1][kW > 1 ? kDv : 4];
+  __shared__ float s_ml[kW][2];
   const int lane = threadIdx.x & 63;
+  const int wave = kW > 1 ? threadIdx.x >> 6 : 0;
+  const int h = kW > 1 ? blockIdx.x : 4 * blockIdx.x + (threadIdx.x >> 6), t = blockIdx.y;
+  if (h >= heads) return;
+  const float sk = sinks != nullptr ? sinks[h] * kLog2e : -INFINITY;
   const int2 rs = ws_rows[t];
   const int splits = rs.y;
-  if (h >= heads || splits <= 1) return;
+  if (splits <= 1) return;
   const int64_t b0 = static_cast<int64_t>(rs.x) * heads + h;
-  // Splits in batches of 8 with every load of a batch issued before any is
+  // Splits in batches with every load of a batch issued before any is
   // used; a running max rescales the partial sums between batches.
-  constexpr int kBatch = 8;
+  constexpr int kBatch = kW > 1 ? 6 : 8;
   float M = -INFINITY, L = 0.0f;
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  for (int s0 = 0; s0 < splits; s0 += kBatch) {
+  for (int s0 = wave; s0 < splits; s0 += kW * kBatch) {
     float ms[kBatch], ls[kBatch];
     float4 v[kBatch][2];
 #pragma unroll
     for (int b = 0; b < kBatch; ++b) {
-      const bool ok = s0 + b < splits;
-      const int64_t row = b0 + static_cast<int64_t>(ok ? s0 + b : s0) * heads;
+      const bool ok = s0 + kW * b < splits;
+      const int64_t row = b0 + static_cast<int64_t>(ok ? s0 + kW * b : s0) * heads;
       const float2 ml = *reinterpret_cast<const float2*>(ws_ml + row * 2);
       ms[b] = ok ? ml.x : -INFINITY;
       ls[b] = ml.y;
@@ -800,10 +811,32 @@ __global__ void __launch_bounds__(256) decode_combine_kernel(
       for (int i = 0; i < 8; ++i) acc[i] += x[i] * f;
     }
   }
+  if constexpr (kW > 1) {  // channels 2 threadIdx.x and the next, in acc[0], acc[1]
+    *reinterpret_cast<float4*>(&s_acc[wave][8 * lane]) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+    *reinterpret_cast<float4*>(&s_acc[wave][8 * lane + 4]) = make_float4(acc[4], acc[5], acc[6], acc[7]);
+    if (lane == 0) {
+      s_ml[wave][0] = M;
+      s_ml[wave][1] = L;
+    }
+    __syncthreads();
+    M = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < kW; ++w) M = fmaxf(M, s_ml[w][0]);
+    L = 0.0f;
+    acc[0] = acc[1] = 0.0f;
+#pragma unroll
+    for (int w = 0; w < kW; ++w) {
+      const float mw = s_ml[w][0];
+      const float f = (mw == -INFINITY) ? 0.0f : exp2f(mw - M);
+      L += s_ml[w][1] * f;
+      const float2 x = *reinterpret_cast<const float2*>(&s_acc[w][2 * threadIdx.x]);
+      acc[0] += x.x * f;
+      acc[1] += x.y * f;
+    }
+  }
   float den = L;
   float numf = 1.0f;
   if (sinks != nullptr) {
-    const float sk = sinks[h] * kLog2e;
     const float Mp = fmaxf(M, sk);
     if (Mp != -INFINITY) {
       numf = (M == -INFINITY) ? 0.0f : exp2f(M - Mp);
@@ -811,14 +844,16 @@ __global__ void __launch_bounds__(256) decode_combine_kernel(
     }
   }
   const float inv = (den > 0.0f) ? numf / den : 0.0f;
-  uint32_t w[4];
+  constexpr int kC = kW > 1 ? 2 : 8;  // channels of a thread
+  uint32_t w[kC / 2];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < kC / 2; ++i)
     w[i] = static_cast<uint32_t>(f32_to_bf16(acc[2 * i] * inv)) |
            (static_cast<uint32_t>(f32_to_bf16(acc[2 * i + 1] * inv)) << 16);
   uint16_t* orow = out + static_cast<int64_t>(t) * out_tok_stride + h * out_head_stride;
-  *reinterpret_cast<uint4*>(orow + 8 * lane) = make_uint4(w[0], w[1], w[2], w[3]);
-  if (lane == 0 && lse != nullptr)
+  if constexpr (kW > 1) *reinterpret_cast<uint32_t*>(orow + 2 * threadIdx.x) = w[0];
+  else *reinterpret_cast<uint4*>(orow + 8 * lane) = make_uint4(w[0], w[1], w[2], w[3]);
+  if (lane == 0 && wave == 0 && lse != nullptr)
     lse[static_cast<int64_t>(t) * lse_stride + h] = (L > 0.0f) ? (M + log2f(L)) * kLn2 : -INFINITY;
 }
 
@@ -899,8 +934,12 @@ extern "C" int ekv_sparse_mla_decode(const uint16_t* q, int64_t q_tok_stride, in
   }
   int rc = ekv_launch_status();
   if (rc) return rc;
-  hipLaunchKernelGGL(decode_combine_kernel, dim3(heads / 4, num_tokens), dim3(256), 0, s, ws_o, ws_ml, ws_rows,
-                     heads, sinks, out, out_tok_stride, out_head_stride, lse, lse_stride);
+  if (groups > 8 * static_cast<int64_t>(num_tokens))  // more than 8 splits a row
+    hipLaunchKernelGGL(decode_combine_kernel<4>, dim3(heads, num_tokens), dim3(256), 0, s, ws_o, ws_ml, ws_rows, heads,
+                       sinks, out, out_tok_stride, out_head_stride, lse, lse_stride);
+  else
+    hipLaunchKernelGGL(decode_combine_kernel<1>, dim3(heads / 4, num_tokens), dim3(256), 0, s, ws_o, ws_ml, ws_rows,
+                       heads, sinks, out, out_tok_stride, out_head_stride, lse, lse_stride);
   return ekv_launch_status();
 }
 
