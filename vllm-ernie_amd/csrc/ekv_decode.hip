@@ -1,6 +1,7 @@
 // Sparse MLA decode over gathered latent rows (DSA top-k + window, HCA
 // compressed + window), with the per-head attention sink in the softmax
-// denominator.
+// denominator.  Calls of many or of short rows take ekv_decode_rows.hip
+// instead.
 //
 // Workgroup = (query row t, split s of its index row): 8 waves, a scorer and
 // a data wave per group of 16 heads, the two waves of a group on one SIMD
@@ -28,7 +29,7 @@
 // O / l in fp32 plus (m, l); the combine kernel merges the splits, adds the
 // sink and writes bf16 out and the natural-log lse (log sum_j exp(s_j), sink
 // excluded).  A row of one split is finished in place.
-#include "ekv_common.h"
+#include "ekv_decode.h"
 #include "ekv_internal.h"
 
 #include <atomic>
@@ -37,48 +38,12 @@
 
 namespace ekv {
 
-constexpr int kDv = 512;
 constexpr int kTile = 32;
 constexpr int kGroups = 4;                   // head groups of 16 (up to 64 heads)
 constexpr int kThreads = 64 * 2 * kGroups;   // a scorer and a data wave per head group
 constexpr int kMaxSplitEntries = 1024;       // index entries one workgroup resolves
 constexpr int kMaxSplitTiles = kMaxSplitEntries / kTile;
 constexpr int kTargetGroups = 256;           // one workgroup per CU
-constexpr int kXcds = 8;                     // workgroup b runs on XCD b % 8
-constexpr float kRescaleSlack = 8.0f;        // log2 units: P <= 2**8 between rescales
-constexpr float kLog2e = 0x1.715476p+0f;
-constexpr float kLn2 = 0x1.62e430p-1f;
-
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef short i16x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) i16x4 lds_i16x4;
-
-struct DecodeArgs {
-  const uint16_t* q;        // [T, H, D] bf16
-  int64_t q_tok_stride, q_head_stride;
-  const uint8_t* cache;     // fp8 pages [num_pages, page_stride] or bf16 rows
-  int64_t page_stride;      // bytes (fp8 layout)
-  int64_t num_rows;         // addressable rows (num_pages * 64), < 2**31
-  const int32_t* indices;   // [T, idx_stride]
-  int64_t idx_stride;
-  int32_t width;            // entries per index row
-  const int32_t* lengths;   // [T] or null
-  const int32_t* block_table;  // logical indices when non-null
-  int64_t bt_stride;
-  const int32_t* req_ids;   // [T] with block_table
-  float scale;              // softmax scale
-  int32_t heads;
-  int32_t rows;             // T
-  int32_t groups;           // G workgroups (a multiple of 8), >= T + T * tiles(width) / 32
-  float* ws_o;              // [G, H, 512] fp32, O / l of workgroup g's split
-  float* ws_ml;             // [G, H, 2] (m in log2 units, l)
-  int2* ws_rows;            // [T] (first workgroup, splits) of each row
-  const float* sinks;       // [H] or null
-  uint16_t* out;            // [T, H, 512] bf16
-  int64_t out_tok_stride, out_head_stride;
-  float* lse;               // [T, H] or null
-  int64_t lse_stride;
-};
 
 // Work split.  Row t has tiles_t = ceil(len_t / 32) tiles and gets
 //   splits_t = max(1, min(tiles_t, 1 + floor((G - T) * tiles_t / total_tiles)))
@@ -87,9 +52,6 @@ struct DecodeArgs {
 // G - T >= total_tiles / 32, every split holds at most 32 tiles
 // (kMaxSplitEntries entries).  Row t's splits are the logical workgroups
 // first_t .. first_t + splits_t - 1 (first_t = sum of the splits before it).
-__device__ __forceinline__ int row_len(const DecodeArgs& a, int t) {
-  return a.lengths ? min(max(a.lengths[t], 0), a.width) : a.width;
-}
 __device__ __forceinline__ int row_splits(int64_t extra, int tiles, int64_t total) {
   const int ns = 1 + (total > 0 ? static_cast<int>((extra * tiles) / total) : 0);
   return max(1, min(tiles, ns));  // never more splits than tiles
@@ -224,37 +186,6 @@ __device__ __forceinline__ int img_off(int r, int c, int h) {
   return r * DecodeSmem<D, BF16>::kRowB + 16 * swz_chunk<D, BF16>(c, r) + 8 * h;
 }
 
-// Four e4m3fn bytes -> four bf16 (exact: every e4m3fn value is a bf16 value).
-__device__ __forceinline__ uint2 fp8x4_bf16(uint32_t w) {
-  const bf16x2 lo = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.0f, false);
-  const bf16x2 hi = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.0f, true);
-  return make_uint2(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi));
-}
-__device__ __forceinline__ bf16x8 fp8x8_bf16(uint2 w) {
-  const uint2 lo = fp8x4_bf16(w.x), hi = fp8x4_bf16(w.y);
-  return __builtin_bit_cast(bf16x8, make_uint4(lo.x, lo.y, hi.x, hi.y));
-}
-
-__device__ __forceinline__ uint32_t bf16x2_bits(float a, float b) {
-  const bf16x2 v = {static_cast<__bf16>(a), static_cast<__bf16>(b)};  // round to nearest even
-  return __builtin_bit_cast(uint32_t, v);
-}
-
-// ds_read_b64_tr_b8: in each row of 16 lanes, lane j receives byte j % 8 of
-// the 8 bytes addressed by lanes j / 8 + 2m (m = 0..7), as byte m.
-typedef int i32x2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ uint2 lds_read_tr8(const uint8_t* p) {
-  const i32x2 v = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
-      (__attribute__((address_space(3))) i32x2*)((__attribute__((address_space(3))) uint8_t*)(p)));
-  return make_uint2(static_cast<uint32_t>(v.x), static_cast<uint32_t>(v.y));
-}
-// ds_read_b64_tr_b16: lane j receives 16-bit element j % 4 of the 8 bytes
-// addressed by lanes j / 4 + 4m (m = 0..3), as element m.
-__device__ __forceinline__ i16x4 lds_read_tr16(const uint8_t* p) {
-  return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-      (lds_i16x4*)((__attribute__((address_space(3))) uint8_t*)(p)));
-}
-
 // Max of v over the lanes l, l ^ 16, l ^ 32, l ^ 48 (the four 16-lane rows),
 // with VALU lane swaps instead of LDS permutes: after a swap of rows r and
 // r ^ 1 (or halves) between two copies of v, the max of the two results is
@@ -266,12 +197,6 @@ __device__ __forceinline__ float max_rows(float v) {
   const uint32_t w = __float_as_uint(m);
   const auto b = __builtin_amdgcn_permlane32_swap(w, w, false, false);
   return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
-
-// s_waitcnt vmcnt(N), other counters untouched.
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
 }
 
 // Data waves: wait until at most n tiles' loads (n < kAhead) are in flight.
@@ -898,7 +823,7 @@ extern "C" int ekv_sparse_mla_decode(const uint16_t* q, int64_t q_tok_stride, in
   EKV_CHECK(num_tokens >= 0 && width >= 0, "sizes must be >= 0");
   if (num_tokens == 0) return 0;
   EKV_CHECK(dim == 512 || dim == 576, "dim must be 512 or 576");
-  EKV_CHECK(heads > 0 && heads % 16 == 0 && heads <= 16 * kGroups, "heads must be a multiple of 16, <= 64");
+  EKV_CHECK(heads > 0 && heads % 16 == 0 && heads <= kMaxHeads, "heads must be a multiple of 16, <= 64");
   EKV_CHECK(q && cache && indices && out, "null pointer");
   EKV_CHECK(block_table == nullptr || req_ids != nullptr, "block_table needs req_ids");
   EKV_CHECK(q_tok_stride % 8 == 0 && q_head_stride % 8 == 0 && aligned16(q), "q must be 16-byte aligned rows");
@@ -924,6 +849,7 @@ extern "C" int ekv_sparse_mla_decode(const uint16_t* q, int64_t q_tok_stride, in
                static_cast<int32_t>(groups), ws_o, ws_ml, ws_rows, sinks, out, out_tok_stride, out_head_stride,
                lse, lse_stride};
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (decode_rows_takes(num_tokens, heads, width)) return launch_decode_rows(a, dim, cache_bf16 != 0, s);
   const dim3 grid(static_cast<uint32_t>(groups));
   if (dim == 576) {
     if (cache_bf16) launch_decode<576, true>(a, grid, s);

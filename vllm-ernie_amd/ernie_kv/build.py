@@ -47,6 +47,7 @@ SOURCES = {
     "ekv_hca.hip": EXACT,
     "ekv_indexer.hip": EXACT + MFMA_VGPR,
     "ekv_decode.hip": [],
+    "ekv_decode_rows.hip": [],
     "ekv_quant.hip": EXACT,
     "ekv_mxfp4.hip": EXACT,
     "ekv_pages.hip": EXACT,
