@@ -1,0 +1,61 @@
+"""The many-row indexer top-k (more rows than the fused launch takes): its
+shared-page filter, its per-row bounds and the select of its candidates give
+the same indices as exact scores of every token and the exact select over
+them, both of which test_gpu_indexer holds against the oracle bit for bit.
+Rows of one request (causal lengths), of several with group boundaries inside
+a workgroup's rows, and of mixed requests; unmapped pages, ties, constant rows
+and rows shorter than k."""
+
+import numpy as np
+import pytest
+import torch
+
+from helpers import to_dev
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(dev, T, n_seqs, order, max_len, kind, seed):
+    from ernie_kv import ops
+
+    rng = np.random.default_rng(seed)
+    g = torch.Generator(device=dev).manual_seed(seed)
+    pages = (max_len + 63) // 64
+    bt = rng.permutation(n_seqs * pages).astype(np.int32).reshape(n_seqs, pages)
+    kcache = torch.zeros((n_seqs * pages, ops.fp8_page_bytes(128)), dtype=torch.uint8, device=dev)
+    n = n_seqs * pages * 64
+    k = torch.randn(n, 128, device=dev, generator=g) * (0.1 + 3 * torch.rand(n, 1, device=dev, generator=g))
+    if kind == "ties":
+        k = k[torch.randint(0, 30, (n,), device=dev, generator=g)]
+    elif kind == "constant":
+        k = k[:1].expand(n, 128)
+    ops.indexer_k_insert(k.bfloat16().contiguous(), torch.arange(n, device=dev), kcache)
+    if kind == "unmapped":
+        bt[:, 1] = -1
+        bt[-1, -1] = n_seqs * pages + 7
+    req = np.sort(rng.integers(0, n_seqs, T)) if order == "runs" else rng.integers(0, n_seqs, T)
+    req = req.astype(np.int32)
+    lengths = np.minimum(max_len, 1 + np.arange(T) % (max_len + 40)).astype(np.int32)
+    q = torch.randn(T, 64, 128, device=dev, generator=g).bfloat16()
+    w = torch.randn(T, 64, device=dev, generator=g).bfloat16()
+    return (*ops.indexer_q_quant(q, w), kcache, to_dev(bt, dev), to_dev(req, dev), to_dev(lengths, dev))
+
+
+@pytest.mark.parametrize("T,n_seqs,order,max_len,k,kind", [
+    (1025, 1, "runs", 900, 64, "normal"),
+    (1100, 3, "runs", 517, 256, "ties"),
+    (1031, 5, "mixed", 640, 64, "normal"),
+    (1040, 1, "runs", 2500, 2048, "unmapped"),
+    (1032, 2, "runs", 700, 500, "constant"),
+])
+def test_many_rows_topk_matches_exact_scores(dev, T, n_seqs, order, max_len, k, kind):
+    from ernie_kv import ops
+
+    q8, w, dig, kcache, bt, req, lengths = _case(dev, T, n_seqs, order, max_len, kind, T + max_len)
+    scores = torch.full((T, max_len), float("nan"), device=dev)
+    ops.indexer_score(dig, w, kcache, bt, req, lengths, max_len, scores)
+    ref = torch.empty((T, k), dtype=torch.int32, device=dev)
+    ops.topk_select(scores, lengths, k, ref)
+    got = torch.empty((T, k), dtype=torch.int32, device=dev)
+    ops.indexer_topk(q8, dig, w, kcache, bt, req, lengths, max_len, got)
+    assert torch.equal(got, ref)

@@ -839,6 +839,342 @@ __global__ void zero_u32_kernel(uint32_t* p, int64_t n) {
 }
 
 // ---------------------------------------------------------------------------
+// Many rows (fp8 keys; prompt chunks): filter and bounds.
+//
+// filter_kernel streams a row's pages for that row alone; a chunk's rows all
+// read the same pages.  Here a workgroup takes kRowsWg consecutive rows, two a
+// wave, and a run of pages, and when the rows are one request's (else each wave
+// streams its rows by itself) every page is loaded once into LDS for all of
+// them.  What is left is VALU work, about 165 instructions per page and row:
+// relu and the weighted sum are 128 of them, the sums over the lane groups 6
+// (lane swaps that also put token l into lane l), the bounds the rest.  No
+// histogram: the bounds kernel reads the stored bounds.
+// 4096 rows ending at 32768: 2.35 -> 1.01 ms (the bounds kernel adds 0.18; the
+// candidates left to score fall from 3100 to about 1800 a row, verify 1.26 ->
+// 0.99 ms, and the select 0.52 -> 0.31).
+//
+// Each token gets one word: U_s (bf16, rounded up) in the high half, L_s (bf16,
+// rounded down) in the low one.
+// ---------------------------------------------------------------------------
+constexpr int kRowsWave = 2;
+constexpr int kRowsWaves = 4;
+constexpr int kRowsWg = kRowsWave * kRowsWaves;
+constexpr int kRowsBufs = 3;                       // LDS page buffers: one in use, two loading
+constexpr int kRowsPage = kIdxPageBytes + 256;     // values, then the 64 scales
+
+// 16-bit key of a bf16 bound (order of score_key; -0 as +0).
+__device__ __forceinline__ uint32_t bound_key(uint32_t bits) {
+  if (bits == 0x8000u) bits = 0u;
+  return (bits & 0x8000u) ? (~bits & 0xffffu) : (bits | 0x8000u);
+}
+
+// Global->LDS loads (lane i's bytes at src to dst + 16 i / 4 i), as asm so
+// that later LDS reads do not wait for them; the caller waits.
+__device__ __forceinline__ void page_load16(const uint8_t* src, const void* dst) {
+  const uint32_t at = static_cast<uint32_t>(
+      reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const uint8_t*)(dst)));
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+               :
+               : "s"(__builtin_amdgcn_readfirstlane(at)), "v"(src)
+               : "m0", "memory");
+}
+__device__ __forceinline__ void page_load4(const uint8_t* src, const void* dst) {
+  const uint32_t at = static_cast<uint32_t>(
+      reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const uint8_t*)(dst)));
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off"
+               :
+               : "s"(__builtin_amdgcn_readfirstlane(at)), "v"(src)
+               : "m0", "memory");
+}
+template <int N>
+__device__ __forceinline__ void wait_vm_at_most() {
+  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
+}
+
+// Sum over the four lane groups of each of a page's four blocks; lane l gets
+// that of token l = 16 b + col.
+__device__ __forceinline__ float page_sums(const float (&acc)[4]) {
+  auto u = [](float f) { return __float_as_uint(f); };
+  auto f = [](uint32_t v) { return __uint_as_float(v); };
+  const auto a = __builtin_amdgcn_permlane32_swap(u(acc[0]), u(acc[2]), false, false);
+  const auto b = __builtin_amdgcn_permlane32_swap(u(acc[1]), u(acc[3]), false, false);
+  const float s02 = f(a[0]) + f(a[1]), s13 = f(b[0]) + f(b[1]);
+  const auto c = __builtin_amdgcn_permlane16_swap(u(s02), u(s13), false, false);
+  return f(c[0]) + f(c[1]);
+}
+
+// The two bounds of a token as one word.
+__device__ __forceinline__ uint32_t bound_word(float sc, float e) {
+  const uint32_t up = bf16_round_up(sc + e);
+  const uint32_t dn = bf16_round_up(-(sc - e)) ^ 0x8000u;
+  return (up << 16) | dn;
+}
+
+struct RowOps {
+  i32x8 qa[kRowsWave][4];
+  float wv[kRowsWave][4][4];
+  float eb[kRowsWave];
+};
+
+// Adds a block's 16 tokens (kv) to the wave's rows' sums.
+__device__ __forceinline__ void row_block(const RowOps& op, int r, const i32x8& kv, float& acc) {
+  acc = 0.0f;
+#pragma unroll
+  for (int hb = 0; hb < 4; ++hb) {
+    const f32x4 cc = filter_mfma(op.qa[r][hb], kv);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc = __builtin_fmaf(op.wv[r][hb][i], relu_bits(cc[i]), acc);
+  }
+}
+
+__global__ void __launch_bounds__(64 * kRowsWaves) __attribute__((amdgpu_waves_per_eu(3)))
+filter_rows_kernel(FilterArgs a, uint32_t* bounds) {
+  __shared__ __align__(16) uint8_t s_page[kRowsBufs][kRowsPage];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = lane >> 4, col = lane & 15;
+  // An XCD (block % 8) takes the runs x of a run of row groups, so a page is
+  // read by neighbouring groups on one XCD at about the same time.
+  const int ngroups = (a.rows + kRowsWg - 1) / kRowsWg;
+  const int per_xcd = (ngroups + 7) / 8;
+  const int slot = static_cast<int>(blockIdx.x) >> 3;
+  const int group = static_cast<int>(blockIdx.x & 7) * per_xcd + slot % per_xcd;
+  const int x = slot / per_xcd;
+  if (group >= ngroups) return;
+  const int t0 = group * kRowsWg;
+
+  // the group's rows: lengths, one request or several
+  int n_max = 0;
+  bool same = true;
+  const int32_t req0 = a.req_ids[t0];
+  for (int i = 0; i < kRowsWg; ++i) {
+    const int t = min(t0 + i, a.rows - 1);
+    const int n = min(a.lengths[t], a.max_len);
+    n_max = max(n_max, n > a.k ? n : 0);  // (a row of at most k tokens needs no filtering)
+    same = same && a.req_ids[t] == req0;
+  }
+  const int np_max = (n_max + kPageTokens - 1) / kPageTokens;
+  const int per = (np_max + a.groups - 1) / a.groups;  // pages of a run
+  const int p_begin = min(x * per, np_max), p_end = min(p_begin + per, np_max);
+  if (p_begin >= p_end) return;
+
+  int n[kRowsWave];
+  RowOps op;
+#pragma unroll
+  for (int r = 0; r < kRowsWave; ++r) {
+    const int t = t0 + kRowsWave * wave + r;
+    const int len = t < a.rows ? min(a.lengths[t], a.max_len) : 0;
+    n[r] = len > a.k ? len : 0;
+    FilterOps f;
+    filter_operands_fp8(a.q_fp8 + static_cast<int64_t>(min(t, a.rows - 1)) * kIdxHeads * kIdxDim,
+                        a.w + static_cast<int64_t>(min(t, a.rows - 1)) * kIdxHeads, g, col, f);
+#pragma unroll
+    for (int hb = 0; hb < 4; ++hb) {
+      op.qa[r][hb] = f.qa[hb];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) op.wv[r][hb][i] = f.wv[hb][i];
+    }
+    op.eb[r] = f.eb[0];
+  }
+  auto word = [&](int r, const float (&acc)[4], float scale) -> uint32_t {
+    return bound_word(page_sums(acc) * scale, scale * op.eb[r]);
+  };
+  auto store = [&](int r, int lp, uint32_t wd) {
+    const int s = lp * kPageTokens + lane;
+    if (s < n[r]) bounds[static_cast<int64_t>(t0 + kRowsWave * wave + r) * a.max_len + s] = wd;
+  };
+
+  if (!same) {  // each wave its rows' pages
+#pragma unroll 1
+    for (int r = 0; r < kRowsWave; ++r) {
+      if (n[r] == 0) continue;
+      const PageSource<false> src(a, a.req_ids[t0 + kRowsWave * wave + r], p_end);
+      const int last = min(p_end, (n[r] + kPageTokens - 1) / kPageTokens);
+      for (int lp = p_begin; lp < last; ++lp) {
+        const int64_t page = src.page_of(lp);
+        uint4 kb[4][2];
+        uint32_t ks;
+        src.load(page, kb, ks);
+        float acc[4];
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          const i32x8 kv = i32x8{static_cast<int>(kb[b][0].x), static_cast<int>(kb[b][0].y),
+                                 static_cast<int>(kb[b][0].z), static_cast<int>(kb[b][0].w),
+                                 static_cast<int>(kb[b][1].x), static_cast<int>(kb[b][1].y),
+                                 static_cast<int>(kb[b][1].z), static_cast<int>(kb[b][1].w)};
+          if (r == 0) row_block(op, 0, kv, acc[b]);
+          else row_block(op, 1, kv, acc[b]);
+        }
+        const float scale = page >= 0 ? __uint_as_float(ks) : 0.0f;
+        if (r == 0) store(0, lp, word(0, acc, scale));
+        else store(1, lp, word(1, acc, scale));
+      }
+    }
+    return;
+  }
+
+  // One request: pages through LDS.  Row r's 16-byte chunk j is stored as
+  // chunk j ^ (r / 2 % 8), which spreads a fragment read (16 rows, four
+  // chunks) evenly over the banks.  Instruction k (of 8) copies rows 8 k ..
+  // 8 k + 7; wave w issues k = w and w + 4, wave 0 also the scales.
+  const int32_t* bt = a.block_table + static_cast<int64_t>(req0) * a.bt_stride;
+  const int lane_off = (lane >> 3) * kIdxDim + 16 * ((lane & 7) ^ ((4 * (wave & 1) + (lane >> 4)) & 7));
+  int32_t ids = 0;       // page ids of logical pages ids0 + lane
+  int ids0 = p_begin - 64;
+  auto page_id = [&](int lp) -> int {  // lp increases from call to call; -1: unmapped
+    if (lp >= ids0 + 64) {
+      ids0 = lp;
+      const int i = lp + lane;
+      ids = (i < p_end && i < a.bt_stride) ? bt[i] : -1;
+      if (ids >= a.num_pages) ids = -1;
+    }
+    return __builtin_amdgcn_readlane(ids, lp - ids0);
+  };
+  auto load = [&](int lp) -> bool {  // true when mapped
+    const int id = page_id(lp);
+    const uint8_t* base = a.kcache + static_cast<int64_t>(max(id, 0)) * a.page_stride;
+    uint8_t* dst = s_page[lp % kRowsBufs];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int k = wave + kRowsWaves * j;
+      page_load16(base + 1024 * k + lane_off, dst + 1024 * k);
+    }
+    if (wave == 0) page_load4(base + kIdxPageBytes + 4 * lane, dst + kIdxPageBytes);
+    return id >= 0;
+  };
+  // A page's words are stored at the start of the next iteration, ahead of the
+  // loads issued there, so that what follows the loads of page p + 1 is known:
+  // the stores of page p - 1 and the loads of page p + 2, which may stay in
+  // flight when page p is done.
+  uint32_t wd[kRowsWave];
+  bool ok0 = load(p_begin), ok1 = p_begin + 1 < p_end ? load(p_begin + 1) : false;
+  wait_vm_at_most<0>();
+  __syncthreads();
+  for (int lp = p_begin; lp < p_end; ++lp) {
+    if (lp > p_begin) {
+#pragma unroll
+      for (int r = 0; r < kRowsWave; ++r) store(r, lp - 1, wd[r]);
+    }
+    const bool more = lp + 2 < p_end;
+    const bool ok2 = more ? load(lp + 2) : false;
+    const uint8_t* pg = s_page[lp % kRowsBufs];
+    const float scale = ok0 ? *reinterpret_cast<const float*>(pg + kIdxPageBytes + 4 * lane) : 0.0f;
+    float acc[kRowsWave][4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      const int row = 16 * b + col, f = (row >> 1) & 7;
+      const uint4 v0 = *reinterpret_cast<const uint4*>(pg + row * kIdxDim + 16 * ((2 * g) ^ f));
+      const uint4 v1 = *reinterpret_cast<const uint4*>(pg + row * kIdxDim + 16 * ((2 * g + 1) ^ f));
+      const i32x8 kv = i32x8{static_cast<int>(v0.x), static_cast<int>(v0.y), static_cast<int>(v0.z),
+                             static_cast<int>(v0.w), static_cast<int>(v1.x), static_cast<int>(v1.y),
+                             static_cast<int>(v1.z), static_cast<int>(v1.w)};
+#pragma unroll
+      for (int r = 0; r < kRowsWave; ++r) row_block(op, r, kv, acc[r][b]);
+    }
+#pragma unroll
+    for (int r = 0; r < kRowsWave; ++r) wd[r] = word(r, acc[r], scale);
+    if (!more) wait_vm_at_most<0>();
+    else if (wave == 0) wait_vm_at_most<3>();
+    else wait_vm_at_most<2>();
+    __syncthreads();
+    ok0 = ok1;
+    ok1 = ok2;
+  }
+#pragma unroll
+  for (int r = 0; r < kRowsWave; ++r) store(r, p_end - 1, wd[r]);
+}
+
+// The row's two thresholds from its bounds, as 16-bit keys: kbound[t] (in the
+// high half, as a score key) of the k-th largest L -- a token whose U is below
+// it has k tokens above it -- and kin[t] of the k-th largest U: fewer than k
+// tokens can reach a token whose L is above it, so it is selected whatever its
+// exact score.  One workgroup per row: the bounds' high 12 key bits, then the
+// low 4 of the two threshold bins.
+__global__ void __launch_bounds__(512) row_bounds_kernel(const uint32_t* bounds, const int32_t* lengths,
+                                                         int32_t max_len, int32_t k, uint32_t* kbound, uint32_t* kin) {
+  __shared__ uint32_t s_hist[2][kHistBins];  // [0] of U, [1] of L
+  __shared__ uint32_t s_low[2][16];
+  __shared__ int s_wave[8];
+  __shared__ int s_res[2];
+  const int tid = threadIdx.x, t = blockIdx.x;
+  const int n = min(lengths[t], max_len);
+  if (n <= k) return;  // unused: every token is selected
+  for (int i = tid; i < 2 * kHistBins; i += 512) s_hist[0][i] = 0;
+  if (tid < 32) s_low[0][tid] = 0;
+  __syncthreads();
+  const uint32_t* row = bounds + static_cast<int64_t>(t) * max_len;
+  constexpr int kPer = 8;
+  for (int i0 = 0; i0 < n; i0 += 512 * kPer) {
+    uint32_t w[kPer];
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      const int i = i0 + 512 * j + tid;
+      w[j] = i < n ? row[i] : 0u;
+    }
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      if (i0 + 512 * j + tid >= n) break;
+      atomicAdd(&s_hist[0][bound_key(w[j] >> 16) >> 4], 1u);
+      atomicAdd(&s_hist[1][bound_key(w[j] & 0xffffu) >> 4], 1u);
+    }
+  }
+  __syncthreads();
+  int bin[2], left[2];  // threshold bin, how many of its keys are needed
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    // 4096 bins, 8 per thread, scanned from the top bin down
+    int c[8];
+    int sum = 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      c[j] = static_cast<int>(s_hist[h][kHistBins - 1 - (8 * tid + j)]);
+      sum += c[j];
+    }
+    int total;
+    int excl = block_scan_excl<512>(sum, s_wave, total);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (excl < k && k <= excl + c[j]) {
+        s_res[0] = kHistBins - 1 - (8 * tid + j);
+        s_res[1] = k - excl;
+      }
+      excl += c[j];
+    }
+    __syncthreads();
+    bin[h] = s_res[0];
+    left[h] = s_res[1];
+    __syncthreads();
+  }
+  for (int i0 = 0; i0 < n; i0 += 512 * kPer) {
+    uint32_t w[kPer];
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      const int i = i0 + 512 * j + tid;
+      w[j] = i < n ? row[i] : 0u;
+    }
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      if (i0 + 512 * j + tid >= n) break;
+      const uint32_t ku = bound_key(w[j] >> 16), kl = bound_key(w[j] & 0xffffu);
+      if (static_cast<int>(ku >> 4) == bin[0]) atomicAdd(&s_low[0][ku & 15u], 1u);
+      if (static_cast<int>(kl >> 4) == bin[1]) atomicAdd(&s_low[1][kl & 15u], 1u);
+    }
+  }
+  __syncthreads();
+  if (tid < 2) {
+    int low = 15, above = 0;
+    for (; low > 0; --low) {
+      const int c = static_cast<int>(s_low[tid][low]);
+      if (left[tid] <= above + c) break;
+      above += c;
+    }
+    const uint32_t key = static_cast<uint32_t>(bin[tid] * 16 + low);
+    if (tid == 0) kin[t] = key;
+    else kbound[t] = key << 16;
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Verify: candidates of a 2048-token chunk, scored exactly into the chunk's
 // slice of the list buffers ([t][chunk0 ...]), count per chunk.
 // ---------------------------------------------------------------------------
@@ -862,12 +1198,17 @@ struct VerifyArgs {
   int32_t chunks;
   const uint8_t* q_fp4;      // fp4 keys: q values [T, 64, 64] (q_digits unused)
   const int32_t* q_scales;   // fp4 keys: [T, 64]
+  const uint32_t* bounds;    // kRows: [T, max_len] words of filter_rows_kernel (upper unused)
+  const uint32_t* kin;       // kRows: [T]
 };
 
 constexpr int kVerifyChunks = 4;  // chunks per verify workgroup
 constexpr int kVerifyPages = kVerifyChunks * kChunk / kPageTokens;
 
-template <bool kFp4>
+// kRows: the bounds are filter_rows_kernel's words, and a candidate whose
+// lower bound is above kin is selected in any case: it is listed with score
+// +inf instead of being scored (about two thirds of a row's candidates).
+template <bool kFp4, bool kRows = false>
 __global__ void __launch_bounds__(256) verify_kernel(VerifyArgs a) {
   __shared__ uint32_t s_table[256];  // fp8: digit table; fp4: q scale words
   __shared__ int16_t s_list[kVerifyChunks * kChunk];  // candidate token offsets in the group, ascending
@@ -921,6 +1262,63 @@ __global__ void __launch_bounds__(256) verify_kernel(VerifyArgs a) {
   const uint32_t kbound = a.kbound[t];
   constexpr int kPer = kChunk / 256;
   const int start = tid * kPer;
+  int total = 0;
+  if constexpr (kRows) {
+    const uint32_t kb16 = kbound >> 16, kin = a.kin[t];
+    uint32_t wd[kVerifyChunks][kPer];
+#pragma unroll
+    for (int cc = 0; cc < kVerifyChunks; ++cc) {
+      const int s0 = (c_begin + cc) * kChunk + start;
+      const bool full = (row & 3) == 0 && s0 + kPer <= n;  // aligned and in bounds
+#pragma unroll
+      for (int j = 0; j < kPer; j += 4) {
+        const uint4 v = full ? *reinterpret_cast<const uint4*>(a.bounds + row + s0 + j) : make_uint4(0, 0, 0, 0);
+        wd[cc][j] = v.x;
+        wd[cc][j + 1] = v.y;
+        wd[cc][j + 2] = v.z;
+        wd[cc][j + 3] = v.w;
+      }
+      if (!full && s0 < n) {
+#pragma unroll
+        for (int j = 0; j < kPer; ++j) wd[cc][j] = s0 + j < n ? a.bounds[row + s0 + j] : 0u;
+      }
+    }
+#pragma unroll
+    for (int cc = 0; cc < kVerifyChunks; ++cc) {
+      const int c = c_begin + cc;
+      const int chunk0 = c * kChunk;
+      const int len = (c < a.chunks) ? max(0, min(kChunk, n - chunk0)) : 0;
+      uint32_t flags = 0, sure = 0;
+#pragma unroll
+      for (int j = 0; j < kPer; ++j) {
+        if (start + j < len && bound_key(wd[cc][j] >> 16) >= kb16) {
+          flags |= 1u << j;
+          if (bound_key(wd[cc][j] & 0xffffu) > kin) sure |= 1u << j;
+        }
+      }
+      // positions in the chunk's list (all candidates) and in the scored list
+      // (those not sure), from one scan; each total is at most 2048
+      int packed;
+      const int ex = block_scan_excl<256>(__popc(flags) | (__popc(flags & ~sure) << 16), s_wave, packed);
+      int slot = ex & 0xffff, pos = total + (ex >> 16);
+#pragma unroll
+      for (int j = 0; j < kPer; ++j)
+        if (flags & (1u << j)) {
+          if (sure & (1u << j)) {
+            const int64_t dst = row + static_cast<int64_t>(c) * kChunk + slot;
+            a.cand_score[dst] = INFINITY;
+            a.cand_idx[dst] = chunk0 + start + j;
+          } else {
+            s_list[pos] = static_cast<int16_t>(chunk0 + start + j - tok0);
+            s_meta[pos] = static_cast<int16_t>((cc << 11) | slot);
+            ++pos;
+          }
+          ++slot;
+        }
+      if (tid == 0 && c < a.chunks) counts[c] = packed & 0xffff;
+      total += packed >> 16;
+    }
+  } else {
   uint4 ub[kVerifyChunks];
 #pragma unroll
   for (int cc = 0; cc < kVerifyChunks; ++cc) {
@@ -934,7 +1332,6 @@ __global__ void __launch_bounds__(256) verify_kernel(VerifyArgs a) {
       ub[cc] = *reinterpret_cast<const uint4*>(tmp);
     }
   }
-  int total = 0;
 #pragma unroll
   for (int cc = 0; cc < kVerifyChunks; ++cc) {
     const int c = c_begin + cc;
@@ -964,6 +1361,7 @@ __global__ void __launch_bounds__(256) verify_kernel(VerifyArgs a) {
       }
     if (tid == 0 && c < a.chunks) counts[c] = ctot;
     total += ctot;
+  }
   }
   __syncthreads();
   if (total == 0) return;
@@ -2416,7 +2814,7 @@ constexpr int kSelPerThread = 8;
 struct SelectArgs {
   const float* scores;       // implicit mode: [T, scores_stride]
   int64_t scores_stride;
-  const int32_t* lengths;    // implicit mode: [T]
+  const int32_t* lengths;    // [T]
   const float* cand_score;   // chunk mode: [T, max_len]
   const int32_t* cand_idx;
   const int32_t* cand_count; // [T, chunks]
@@ -2427,6 +2825,7 @@ struct SelectArgs {
   int64_t out_stride;
   int32_t k;
   int32_t max_len;
+  int32_t sure;              // chunk mode: a score of +inf is a token selected in any case
   int32_t seg_groups;        // chunk mode: 0 = lists of kChunk-token chunks, else of
                              // filter_verify_kernel segments (`seg_groups` per row)
   // Optional merged output (merge_swa_topk of the result): [T, merged_stride]
@@ -2500,9 +2899,33 @@ __global__ void __launch_bounds__(kSelThreads) topk_select_kernel(SelectArgs a) 
     out[pos] = v;
     if (merged && pos < m_topk) merged[pos] = to_merged(v);
   };
+  auto emit_window = [&] {
+    if (!merged) return;
+    const int64_t w = min(seq, static_cast<int64_t>(a.window));
+    for (int64_t c = m_topk + tid; c < a.merged_width; c += kSelThreads)
+      merged[c] = (c < m_topk + w) ? to_merged(seq - w + (c - m_topk)) : -1;
+  };
+
+  // A row of at most k tokens: all of them, in order (2331 rows of a prompt's
+  // start: 75 us through the lists).
+  const int n_row = max(0, min(a.lengths[t], a.max_len));
+  if (n_row <= k) {
+    if (mbt) {
+#pragma unroll
+      for (int j = 0; j < kSelBtPages / kSelThreads; ++j) s_hist[tid + kSelThreads * j] = static_cast<uint32_t>(btv[j]);
+      __syncthreads();
+    }
+    for (int i = tid; i < k; i += kSelThreads) emit(i, i < n_row ? i : -1);
+    emit_window();
+    return;
+  }
 
   // gather the elements; lo / hi track the range of the keys put in LDS
   uint32_t lo = 0xffffffffu, hi = 0u;
+  // The key of sure tokens (0: none): they are above the threshold and take no
+  // part in the passes that look for it.
+  const uint32_t sure_key = a.sure ? score_key(INFINITY) : 0u;
+  int sure = 0;  // this thread's
   int n;
   const float* gsc = nullptr;     // global scores (implicit mode or spilled lists)
   const int32_t* gidx = nullptr;  // global indices (spilled lists); null = implicit
@@ -2573,12 +2996,15 @@ __global__ void __launch_bounds__(kSelThreads) topk_select_kernel(SelectArgs a) 
       for (int q = 0; q < kGather; ++q) {
         const int p = p0 + q * kSelThreads + tid;
         if (p >= n) continue;
-        if (in_lds) {
-          const uint32_t key = score_key(sv[q] + 0.0f);
-          s_key[p] = key;
-          s_idx[p] = iv[q];
+        const uint32_t key = score_key(sv[q] + 0.0f);
+        if (sure_key != 0u && key == sure_key) ++sure;
+        else if (in_lds) {
           lo = min(lo, key);
           hi = max(hi, key);
+        }
+        if (in_lds) {
+          s_key[p] = key;
+          s_idx[p] = iv[q];
         } else {
           st_sc[p] = sv[q];
           st_ix[p] = iv[q];
@@ -2594,12 +3020,20 @@ __global__ void __launch_bounds__(kSelThreads) topk_select_kernel(SelectArgs a) 
   for (int off = 32; off > 0; off >>= 1) {
     lo = min(lo, static_cast<uint32_t>(__shfl_xor(static_cast<int>(lo), off)));
     hi = max(hi, static_cast<uint32_t>(__shfl_xor(static_cast<int>(hi), off)));
+    sure += __shfl_xor(sure, off);
   }
   if ((tid & 63) == 0) {
     sm.wmin[tid >> 6] = lo;
     sm.wmax[tid >> 6] = hi;
+    sm.wave[tid >> 6] = sure;
   }
   __syncthreads();
+  if (sure_key != 0u) {
+    sure = 0;
+#pragma unroll
+    for (int w = 0; w < kSelThreads / 64; ++w) sure += sm.wave[w];
+    __syncthreads();
+  }
   auto key_at = [&](int i) -> uint32_t { return in_lds ? s_key[i] : score_key(gsc[i] + 0.0f); };
   auto idx_at = [&](int i) -> int32_t { return in_lds ? s_idx[i] : (gidx ? gidx[i] : i); };
 
@@ -2622,7 +3056,7 @@ __global__ void __launch_bounds__(kSelThreads) topk_select_kernel(SelectArgs a) 
     const int common = (kmin == kmax) ? 32 : __clz(static_cast<int>(kmin ^ kmax));
     uint32_t mask = common == 0 ? 0u : (common == 32 ? 0xffffffffu : 0xffffffffu << (32 - common));
     uint32_t prefix = kmin & mask;
-    int remaining = k;
+    int remaining = k - sure;
     int top = 32 - common;  // bits [0, top) are still open
     bool first = true;      // the first pass's key range is [kmin, kmax]
     while (top > 0) {
@@ -2643,7 +3077,7 @@ __global__ void __launch_bounds__(kSelThreads) topk_select_kernel(SelectArgs a) 
           int bin = -1;
           if (i < n) {
             const uint32_t key = key_at(i);
-            if ((key & mask) == prefix) {
+            if ((key & mask) == prefix && (sure_key == 0u || key != sure_key)) {
               bin = static_cast<int>((key >> sh) & static_cast<uint32_t>(nb - 1));
               plo = min(plo, key);
               phi = max(phi, key);
@@ -2693,7 +3127,7 @@ __global__ void __launch_bounds__(kSelThreads) topk_select_kernel(SelectArgs a) 
             bool hit = false;
             if (i < n) {
               key = key_at(i);
-              hit = (key & mask) == prefix;
+              hit = (key & mask) == prefix && (sure_key == 0u || key != sure_key);
             }
             const uint64_t bal = __ballot(hit);
             if (bal != 0) {  // wave-uniform
@@ -2786,11 +3220,7 @@ __global__ void __launch_bounds__(kSelThreads) topk_select_kernel(SelectArgs a) 
     eq_base += packed_total >> 16;
   }
   for (int i = gt_base + min(eq_base, need) + tid; i < k; i += kSelThreads) emit(i, -1);
-  if (merged) {
-    const int64_t w = min(seq, static_cast<int64_t>(a.window));
-    for (int64_t c = m_topk + tid; c < a.merged_width; c += kSelThreads)
-      merged[c] = (c < m_topk + w) ? to_merged(seq - w + (c - m_topk)) : -1;
-  }
+  emit_window();
 }
 
 }  // namespace ekv
@@ -2812,6 +3242,7 @@ int num_chunks(int32_t max_len) { return max_len > 0 ? (max_len + kChunk - 1) / 
 // streaming many pages.
 constexpr int64_t kFilterTargetGroups = 768;
 constexpr int64_t kFilterMaxWavePages = 64;
+constexpr int64_t kRowsMin = 256;  // rows from which an unfused call takes filter_rows_kernel
 
 // Count slots [T, groups] of either path: chunks per row, or segments (at most
 // ceil(kFilterTargetGroups / T) per row).
@@ -2864,6 +3295,7 @@ TopkWorkspace carve(void* workspace, int64_t T, int64_t L) {
 // a top-k call make the same plan.
 struct FilterPlan {
   bool fused;
+  bool rows;        // unfused: filter_rows_kernel and row_bounds_kernel (groups: runs of pages per row)
   int waves;        // fused: waves per workgroup (12 or 4)
   int groups;       // workgroups per row
   int stage_pages;  // fused: LDS pages per workgroup
@@ -2903,7 +3335,7 @@ bool plan_fused(int64_t T, int32_t max_len, int64_t pages, int cus, int64_t targ
     if (smem > kLdsPerCu) return false;
     const int64_t capacity = static_cast<int64_t>(occupancy(kernel, 64 * kWaves, smem)) * cus;
     if (T * groups <= capacity && T * groups <= count_slots(T, max_len)) {
-      p = FilterPlan{true, kWaves, static_cast<int>(groups), stage, smem};
+      p = FilterPlan{true, false, kWaves, static_cast<int>(groups), stage, smem};
       return true;
     }
     groups = capacity / T;
@@ -2914,7 +3346,7 @@ bool plan_fused(int64_t T, int32_t max_len, int64_t pages, int cus, int64_t targ
 template <bool kFp4>
 FilterPlan plan_filter(int64_t T, int32_t max_len) {
   const int64_t pages = (static_cast<int64_t>(max_len) + kPageTokens - 1) / kPageTokens;
-  FilterPlan p{false, 4, 1, 0, 0};
+  FilterPlan p{false, false, 4, 1, 0, 0};
   // unfused: about kFilterTargetGroups workgroups over T equal rows, and at
   // least enough that a max_len row takes at most kFilterMaxWavePages pages
   // per wave (rows of mixed lengths use slots in proportion to their pages);
@@ -2928,6 +3360,14 @@ FilterPlan plan_filter(int64_t T, int32_t max_len) {
     return p;
   if (T <= cus && plan_fused<12, kFp4>(T, max_len, pages, cus, cus, p)) return p;
   if (plan_fused<4, kFp4>(T, max_len, pages, cus, kFilterTargetGroups, p)) return p;
+  if (!kFp4 && T >= kRowsMin) {
+    // three workgroups a CU, each a run of pages of kRowsWg rows, about four
+    // rounds of them so that the last is short
+    const int64_t row_groups = (T + kRowsWg - 1) / kRowsWg;
+    p.rows = true;
+    p.groups = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>((pages + 7) / 8,
+                                                                       (12 * cus + row_groups - 1) / row_groups)));
+  }
   return p;
 }
 
@@ -3006,7 +3446,7 @@ extern "C" int ekv_topk_select(const float* scores, int64_t scores_stride, const
   EKV_CHECK(out_stride >= k, "out_stride must be >= k");
   EKV_CHECK(max_len >= 0 && scores_stride >= max_len, "scores_stride must be >= max_len");
   SelectArgs s{scores, scores_stride, lengths, nullptr, nullptr, nullptr, 0, nullptr, nullptr, out, out_stride, k,
-               max_len, 0, nullptr, 0, 0, nullptr, 0, nullptr, 0, nullptr, 0};
+               max_len, 0, 0, nullptr, 0, 0, nullptr, 0, nullptr, 0, nullptr, 0};
   launch_select(s, num_tokens, static_cast<hipStream_t>(stream));
   return ekv_launch_status();
 }
@@ -3095,6 +3535,13 @@ int run_filter(const TopkQuery& q, const uint8_t* kcache, int64_t page_stride, i
       hipLaunchKernelGGL((filter_verify_kernel<12, kFp4>), grid, dim3(64 * 12), plan.smem, s, fa);
     else
       hipLaunchKernelGGL((filter_verify_kernel<4, kFp4>), grid, dim3(64 * 4), plan.smem, s, fa);
+  } else if (plan.rows && max_len > 0) {
+    const int64_t row_groups = (T + kRowsWg - 1) / kRowsWg;
+    uint32_t* bounds = reinterpret_cast<uint32_t*>(ws.upper);  // (4 bytes an entry are reserved)
+    hipLaunchKernelGGL(filter_rows_kernel, dim3(static_cast<unsigned>(8 * ((row_groups + 7) / 8) * plan.groups)),
+                       dim3(64 * kRowsWaves), 0, s, f, bounds);
+    hipLaunchKernelGGL(row_bounds_kernel, dim3(num_tokens), dim3(512), 0, s, bounds, lengths, max_len, k, ws.kbound,
+                       ws.arrive);
   } else if (max_len > 0) {
     const int64_t nz = T * kHistBins + 2 * T;  // this call's hist, arrive, kbound
     const int64_t zero_blocks = (nz + 255) / 256;
@@ -3132,13 +3579,17 @@ int run_select(const TopkQuery& q, const uint8_t* kcache, int64_t page_stride, i
   if (!plan.fused) {
     VerifyArgs v{q.q_digits, q.w, kcache, page_stride, num_pages, block_table, bt_stride, req_ids, lengths,
                  max_len, k, ws.upper, ws.kbound, ws.cand_score, ws.cand_idx, ws.counts, chunks,
-                 kFp4 ? q.q : nullptr, q.q_scales};
-    hipLaunchKernelGGL(verify_kernel<kFp4>, dim3((chunks + kVerifyChunks - 1) / kVerifyChunks, num_tokens),
-                       dim3(256), 0, s, v);
+                 kFp4 ? q.q : nullptr, q.q_scales, reinterpret_cast<const uint32_t*>(ws.upper), ws.arrive};
+    const dim3 grid((chunks + kVerifyChunks - 1) / kVerifyChunks, num_tokens);
+    if (plan.rows && max_len > 0) {
+      if constexpr (!kFp4) hipLaunchKernelGGL((verify_kernel<false, true>), grid, dim3(256), 0, s, v);
+    } else {
+      hipLaunchKernelGGL(verify_kernel<kFp4>, grid, dim3(256), 0, s, v);
+    }
   }
   SelectArgs sel{nullptr, 0, lengths, ws.cand_score, ws.cand_idx, ws.counts, plan.fused ? plan.groups : chunks,
                  ws.stage_score, ws.stage_idx, topk_out, out_stride, k, static_cast<int32_t>(L),
-                 plan.fused ? plan.groups : 0, merged_out, merged_stride, merged_width, positions, window,
+                 plan.rows ? 1 : 0, plan.fused ? plan.groups : 0, merged_out, merged_stride, merged_width, positions, window,
                  merged_slots ? block_table : nullptr, bt_stride, req_ids, num_pages};
   launch_select(sel, num_tokens, s);
   return ekv_launch_status();
@@ -3300,7 +3751,7 @@ extern "C" int ekv_dsa_decode_prologue_topk_merged(
   EKV_CHECK(num_tokens >= 0 && window >= 0 && max_len >= 0 && k_top > 0, "bad sizes");
   if (num_tokens == 0) return 0;
   const int64_t T = num_tokens;
-  FilterPlan plan{false, 4, 1, 0, 0};
+  FilterPlan plan{false, false, 4, 1, 0, 0};
   // folded only when no row can score a key this call appends: every
   // sequence's new rows (its last positions) number at most `window`
   if (heads == kIdxHeads && max_new_rows >= 1 && max_new_rows <= window && merged_out != nullptr)
