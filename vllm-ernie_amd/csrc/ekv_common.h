@@ -89,6 +89,34 @@ __device__ __forceinline__ void fp8x4_to_bf16x4(uint32_t w, uint32_t& lo, uint32
   hi = __builtin_amdgcn_perm(__float_as_uint(b[1]), __float_as_uint(b[0]), 0x07060302u);
 }
 
+// s_waitcnt vmcnt(N), other counters untouched.
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
+}
+
+// Direct global->LDS loads: lane i's 16 (4) bytes at src to dst + 16 i (4 i),
+// dst wave-uniform.  Written as asm because the compiler, which tracks the
+// builtin's LDS write but not which bytes it covers, waits for it before every
+// later LDS read (vmcnt(0), a whole memory latency); the caller waits
+// (wait_vm) before the barrier that hands the bytes on.
+__device__ __forceinline__ void load_lds16(const void* src, const void* dst) {
+  const uint32_t at =
+      static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const uint8_t*)(dst)));
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+               :
+               : "s"(__builtin_amdgcn_readfirstlane(at)), "v"(src)
+               : "m0", "memory");
+}
+__device__ __forceinline__ void load_lds4(const void* src, const void* dst) {
+  const uint32_t at =
+      static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const uint8_t*)(dst)));
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off"
+               :
+               : "s"(__builtin_amdgcn_readfirstlane(at)), "v"(src)
+               : "m0", "memory");
+}
+
 // Order-preserving uint32 key of an fp32 score (larger score -> larger key).
 __device__ __forceinline__ uint32_t score_key(float s) {
   uint32_t u = __float_as_uint(s);

@@ -80,12 +80,6 @@ __device__ __forceinline__ i16x4 lds_read_tr16(const uint8_t* p) {
       (lds_i16x4*)((__attribute__((address_space(3))) uint8_t*)(p)));
 }
 
-// s_waitcnt vmcnt(N), other counters untouched.
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
-}
-
 // The whole-row kernel (ekv_decode_rows.hip): whether a call of num_tokens rows
 // of `width` entries takes it, and its launch.
 bool decode_rows_takes(int32_t num_tokens, int32_t heads, int32_t width);

@@ -129,30 +129,6 @@ __device__ __forceinline__ float max_halves(float v) {
   return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
 
-// Direct global->LDS load: lane i's 16 bytes at src to dst + 16 i (dst wave-
-// uniform).  Written as asm because the compiler, which tracks the builtin's
-// LDS write but not which bytes it covers, waits for it before every later
-// LDS read (vmcnt(0), a whole memory latency per step); the caller waits
-// (wait_vm) before the barrier that hands the bytes on.
-__device__ __forceinline__ void load_lds16(const uint8_t* src, uint8_t* dst) {
-  const uint32_t at = static_cast<uint32_t>(
-      reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)(dst)));
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-               :
-               : "s"(__builtin_amdgcn_readfirstlane(at)), "v"(src)
-               : "m0", "memory");
-}
-
-// The same for 4 bytes a lane.
-__device__ __forceinline__ void load_lds4(const uint8_t* src, uint8_t* dst) {
-  const uint32_t at = static_cast<uint32_t>(
-      reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)(dst)));
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off"
-               :
-               : "s"(__builtin_amdgcn_readfirstlane(at)), "v"(src)
-               : "m0", "memory");
-}
-
 // Row (of 16) of k-slot m (0..7) of half-wave hl in the S^T accumulators / the
 // V^T P^T operands.
 __device__ __forceinline__ int slot_row(int hl, int m) { return m < 4 ? 4 * hl + m : 8 + 4 * hl + (m - 4); }

@@ -868,29 +868,6 @@ __device__ __forceinline__ uint32_t bound_key(uint32_t bits) {
   return (bits & 0x8000u) ? (~bits & 0xffffu) : (bits | 0x8000u);
 }
 
-// Global->LDS loads (lane i's bytes at src to dst + 16 i / 4 i), as asm so
-// that later LDS reads do not wait for them; the caller waits.
-__device__ __forceinline__ void page_load16(const uint8_t* src, const void* dst) {
-  const uint32_t at = static_cast<uint32_t>(
-      reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const uint8_t*)(dst)));
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-               :
-               : "s"(__builtin_amdgcn_readfirstlane(at)), "v"(src)
-               : "m0", "memory");
-}
-__device__ __forceinline__ void page_load4(const uint8_t* src, const void* dst) {
-  const uint32_t at = static_cast<uint32_t>(
-      reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const uint8_t*)(dst)));
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off"
-               :
-               : "s"(__builtin_amdgcn_readfirstlane(at)), "v"(src)
-               : "m0", "memory");
-}
-template <int N>
-__device__ __forceinline__ void wait_vm_at_most() {
-  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
-}
-
 // Sum over the four lane groups of each of a page's four blocks; lane l gets
 // that of token l = 16 b + col.
 __device__ __forceinline__ float page_sums(const float (&acc)[4]) {
@@ -1037,9 +1014,9 @@ filter_rows_kernel(FilterArgs a, uint32_t* bounds) {
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int k = wave + kRowsWaves * j;
-      page_load16(base + 1024 * k + lane_off, dst + 1024 * k);
+      load_lds16(base + 1024 * k + lane_off, dst + 1024 * k);
     }
-    if (wave == 0) page_load4(base + kIdxPageBytes + 4 * lane, dst + kIdxPageBytes);
+    if (wave == 0) load_lds4(base + kIdxPageBytes + 4 * lane, dst + kIdxPageBytes);
     return id >= 0;
   };
   // A page's words are stored at the start of the next iteration, ahead of the
@@ -1048,7 +1025,7 @@ filter_rows_kernel(FilterArgs a, uint32_t* bounds) {
   // flight when page p is done.
   uint32_t wd[kRowsWave];
   bool ok0 = load(p_begin), ok1 = p_begin + 1 < p_end ? load(p_begin + 1) : false;
-  wait_vm_at_most<0>();
+  wait_vm<0>();
   __syncthreads();
   for (int lp = p_begin; lp < p_end; ++lp) {
     if (lp > p_begin) {
@@ -1073,9 +1050,9 @@ filter_rows_kernel(FilterArgs a, uint32_t* bounds) {
     }
 #pragma unroll
     for (int r = 0; r < kRowsWave; ++r) wd[r] = word(r, acc[r], scale);
-    if (!more) wait_vm_at_most<0>();
-    else if (wave == 0) wait_vm_at_most<3>();
-    else wait_vm_at_most<2>();
+    if (!more) wait_vm<0>();
+    else if (wave == 0) wait_vm<3>();
+    else wait_vm<2>();
     __syncthreads();
     ok0 = ok1;
     ok1 = ok2;

@@ -13,12 +13,17 @@
 //    inverse RoPE of the interleaved rope pairs (channels nope_dim ..), and a
 //    UE8M0 fp8 quant per (head, 128 channels), written as
 //    [group][token][head in group * 512 + channel] with exponent byte c of
-//    scale int32 [group][head in group][token] for chunk c.  Four waves, wave
-//    w = channels [128 w, 128 w + 128): Y^T = O^T M^T on
+//    scale int32 [group][head in group][token] for chunk c.  Eight waves, wave
+//    (c, hh) = channels [128 c, +128) of heads [32 hh, +32): Y^T = O^T M^T on
 //    v_mfma_f32_16x16x32_bf16 with A = O^T read from the token's rows in LDS
 //    by transposing reads (ds_read_b64_tr_b16) and B = M^T rows from
-//    registers; a lane's accumulator holds 4 consecutive channels of one
-//    head, so a rope pair never leaves its lane.
+//    registers.  Row 4 kg + i of block cb is channel 32 kg + 4 cb + i of the
+//    wave's, so a lane's accumulators are 32 consecutive channels of a head: a
+//    rope pair never leaves its lane, and the lane stores whole 16-byte runs.
+//    One workgroup a CU walks over tokens with the next token's rows loading
+//    straight into the other LDS buffer: HBM-bound work (96 KB a token), which
+//    two workgroups of four waves that loaded, multiplied and stored in turn
+//    left idle two thirds of the time (2048 tokens: 85 -> 45 us).
 #include "ekv_common.h"
 #include "ekv_internal.h"
 
@@ -118,54 +123,76 @@ struct VhaArgs {
   int32_t heads_per_group, nope_dim, half_rope;
   uint8_t* out;             // [G, T, heads_per_group * 512] fp8
   uint8_t* scale;           // [G, heads_per_group, aligned_tokens] int32, as bytes
+  bool out16;               // out is 16-byte aligned (4-byte stores otherwise)
 };
 
-constexpr int kVhaLds = kVhaHeads * kVhaRowB;
+// Two buffers of a token's 64 rows and of its cos | sin row.
+struct VhaSmem {
+  __align__(16) uint8_t o[2][kVhaHeads * kVhaRowB];
+  __align__(16) float cs[2][kVhaDim];
+};
+constexpr int kVhaWaves = 8;
+constexpr int kVhaGrid = 256;  // one workgroup a CU
 
-__global__ void __launch_bounds__(256) vha_inv_rope_quant_kernel(VhaArgs a) {
-  extern __shared__ __align__(16) uint8_t s_o[];  // kVhaLds bytes: the token's 64 rows
+__global__ void __launch_bounds__(64 * kVhaWaves) vha_inv_rope_quant_kernel(VhaArgs a) {
+  extern __shared__ __align__(16) uint8_t smem_raw[];
+  VhaSmem& sm = *reinterpret_cast<VhaSmem*>(smem_raw);
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // channel chunk
+  const int w8 = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = w8 & 3, hh = w8 >> 2;  // channel chunk, head half
   const int kg = lane >> 4, col = lane & 15;
-  // B = M^T (input heads x output heads): lane (head 16 hb + col, kg) holds
-  // M[head][32 ks + 8 kg .. +7]
-  bf16x8 mb[4][2];
-#pragma unroll
-  for (int hb = 0; hb < 4; ++hb)
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-      mb[hb][ks] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(a.mix + (16 * hb + col) * kVhaHeads +
-                                                                               32 * ks + 8 * kg));
-  for (int tok = blockIdx.x; tok < a.aligned_tokens; tok += gridDim.x) {
-    if (tok >= a.num_tokens) {  // padding rows of the scale buffer: zero bytes
+  // padding rows of the scale buffer: zero bytes
+  if (tid < 4 * kVhaHeads) {
+    for (int tok = a.num_tokens + blockIdx.x; tok < a.aligned_tokens; tok += gridDim.x) {
       const int h = tid >> 2, c = tid & 3;
       const int grp = h / a.heads_per_group, hig = h % a.heads_per_group;
       a.scale[((static_cast<int64_t>(grp) * a.heads_per_group + hig) * a.aligned_tokens + tok) * 4 + c] = 0;
-      continue;
     }
-    __syncthreads();  // the previous token's reads of s_o are done
-    // the token's 64 x 512 bf16 rows into LDS (16-byte loads)
+  }
+  // B = M^T (input heads x output heads): lane (head 32 hh + 16 hb + col, kg)
+  // holds M[head][32 ks + 8 kg .. +7]
+  bf16x8 mb[2][2];
 #pragma unroll
-    for (int j = 0; j < (kVhaHeads * kVhaDim * 2 / 16) / 256; ++j) {
-      const int idx = tid + 256 * j;
-      const int h = idx >> 6, part = idx & 63;
-      const uint4 v = *reinterpret_cast<const uint4*>(a.o + static_cast<int64_t>(tok) * a.o_tok_stride +
-                                                      h * a.o_head_stride + 8 * part);
-      *reinterpret_cast<uint4*>(s_o + h * kVhaRowB + 16 * part) = v;
+  for (int hb = 0; hb < 2; ++hb)
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+      mb[hb][ks] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(a.mix + (32 * hh + 16 * hb + col) * kVhaHeads +
+                                                                               32 * ks + 8 * kg));
+  // A token's rows (one instruction a row) and its 2 half_rope cos | sin values.
+  auto load = [&](int tok, int buf) {
+    const uint16_t* row = a.o + static_cast<int64_t>(tok) * a.o_tok_stride + 8 * lane;
+#pragma unroll
+    for (int j = 0; j < kVhaHeads / kVhaWaves; ++j) {
+      const int h = w8 + kVhaWaves * j;
+      load_lds16(row + h * a.o_head_stride, sm.o[buf] + h * kVhaRowB);
     }
-    __syncthreads();
-    // Y^T[channel][head] for this wave's 8 channel blocks x 4 head blocks
-    f32x4 acc[4][8];
+    if (64 * w8 < 2 * a.half_rope) {
+      const int64_t pos = *(const __attribute__((address_space(4))) int64_t*)(a.positions + tok);  // (scalar load)
+      if (64 * w8 + lane < 2 * a.half_rope)
+        load_lds4(a.cos_sin + pos * a.cs_stride + 64 * w8 + lane, sm.cs[buf] + 64 * w8);
+    }
+  };
+  int tok = blockIdx.x;
+  if (tok >= a.num_tokens) return;
+  load(tok, 0);
+  wait_vm<0>();
+  __syncthreads();
+  for (int it = 0; tok < a.num_tokens; tok += gridDim.x, ++it) {
+    const uint8_t* s_o = sm.o[it & 1];
+    const float* s_cs = sm.cs[it & 1];
+    if (tok + static_cast<int>(gridDim.x) < a.num_tokens) load(tok + gridDim.x, (it + 1) & 1);
+    // Y^T[channel][head] for this wave's 8 channel blocks x 2 head blocks
+    f32x4 acc[2][8];
 #pragma unroll
-    for (int hb = 0; hb < 4; ++hb)
+    for (int hb = 0; hb < 2; ++hb)
 #pragma unroll
       for (int cb = 0; cb < 8; ++cb) acc[hb][cb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int cb = 0; cb < 8; ++cb) {
-      const int ch = 128 * wave + 16 * cb + 4 * (col & 3);
+      const int ch = 128 * wave + 32 * (col & 3) + 4 * cb;
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) {
-        // A = O^T: element m of read h2 is O[32 ks + 8 kg + 4 h2 + m][16 cb + (this lane's column)]
+        // A = O^T: element m of read h2 is O[32 ks + 8 kg + 4 h2 + m][the channel of row `col` of block cb]
         const int r0 = 32 * ks + 8 * kg + (col >> 2);
         const q_i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
             (q_lds_i16x4*)((__attribute__((address_space(3))) uint8_t*)(s_o + r0 * kVhaRowB + 2 * ch)));
@@ -174,23 +201,22 @@ __global__ void __launch_bounds__(256) vha_inv_rope_quant_kernel(VhaArgs a) {
         const q_i16x4 both[2] = {lo, hi};
         const bf16x8 av = __builtin_bit_cast(bf16x8, both);
 #pragma unroll
-        for (int hb = 0; hb < 4; ++hb) acc[hb][cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, mb[hb][ks], acc[hb][cb], 0, 0, 0);
+        for (int hb = 0; hb < 2; ++hb) acc[hb][cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, mb[hb][ks], acc[hb][cb], 0, 0, 0);
       }
     }
-    // lane: head h = 16 hb + col, channels 128 wave + 16 cb + 4 kg + i
-    const int64_t pos = a.positions[tok];
+    // lane: head h = 32 hh + 16 hb + col, channels 128 wave + 32 kg + 4 cb + i
 #pragma unroll
     for (int cb = 0; cb < 8; ++cb) {
-      const int c0 = 128 * wave + 16 * cb + 4 * kg;
+      const int c0 = 128 * wave + 32 * kg + 4 * cb;
       if (c0 + 3 >= a.nope_dim) {  // inverse rotation of the pairs (c0, c0+1), (c0+2, c0+3)
 #pragma unroll
         for (int pr = 0; pr < 2; ++pr) {
           const int c = c0 + 2 * pr;
           if (c < a.nope_dim) continue;
           const int r = (c - a.nope_dim) >> 1;
-          const float cs = a.cos_sin[pos * a.cs_stride + r], sn = a.cos_sin[pos * a.cs_stride + a.half_rope + r];
+          const float cs = s_cs[r], sn = s_cs[a.half_rope + r];
 #pragma unroll
-          for (int hb = 0; hb < 4; ++hb) {
+          for (int hb = 0; hb < 2; ++hb) {
             const float ev = acc[hb][cb][2 * pr], od = acc[hb][cb][2 * pr + 1];
             acc[hb][cb][2 * pr] = ev * cs + od * sn;
             acc[hb][cb][2 * pr + 1] = od * cs - ev * sn;
@@ -198,8 +224,10 @@ __global__ void __launch_bounds__(256) vha_inv_rope_quant_kernel(VhaArgs a) {
         }
       }
     }
+    // the next token's rows have landed (before the stores below are counted)
+    wait_vm<0>();
 #pragma unroll
-    for (int hb = 0; hb < 4; ++hb) {
+    for (int hb = 0; hb < 2; ++hb) {
       float amax = 0.0f;
 #pragma unroll
       for (int cb = 0; cb < 8; ++cb)
@@ -209,20 +237,28 @@ __global__ void __launch_bounds__(256) vha_inv_rope_quant_kernel(VhaArgs a) {
       amax = fmaxf(amax, __shfl_xor(amax, 32));
       const int e = ue8m0_exponent(amax);
       const float inv = exp2i(-e);
-      const int h = 16 * hb + col;
+      const int h = 32 * hh + 16 * hb + col;
       const int grp = h / a.heads_per_group, hig = h % a.heads_per_group;
       uint8_t* orow = a.out + (static_cast<int64_t>(grp) * a.num_tokens + tok) * (a.heads_per_group * kVhaDim) +
                       hig * kVhaDim;
+      uint32_t wd[8];
 #pragma unroll
-      for (int cb = 0; cb < 8; ++cb) {
-        const uint32_t w01 = f32x2_to_fp8(acc[hb][cb][0] * inv, acc[hb][cb][1] * inv);
-        const uint32_t w23 = f32x2_to_fp8(acc[hb][cb][2] * inv, acc[hb][cb][3] * inv);
-        *reinterpret_cast<uint32_t*>(orow + 128 * wave + 16 * cb + 4 * kg) = w01 | (w23 << 16);
+      for (int cb = 0; cb < 8; ++cb)
+        wd[cb] = f32x2_to_fp8(acc[hb][cb][0] * inv, acc[hb][cb][1] * inv) |
+                 (f32x2_to_fp8(acc[hb][cb][2] * inv, acc[hb][cb][3] * inv) << 16);
+      uint8_t* at = orow + 128 * wave + 32 * kg;
+      if (a.out16) {
+        *reinterpret_cast<uint4*>(at) = make_uint4(wd[0], wd[1], wd[2], wd[3]);
+        *reinterpret_cast<uint4*>(at + 16) = make_uint4(wd[4], wd[5], wd[6], wd[7]);
+      } else {
+#pragma unroll
+        for (int cb = 0; cb < 8; ++cb) *reinterpret_cast<uint32_t*>(at + 4 * cb) = wd[cb];
       }
       if (kg == 0)
         a.scale[((static_cast<int64_t>(grp) * a.heads_per_group + hig) * a.aligned_tokens + tok) * 4 + wave] =
             static_cast<uint8_t>(e + 127);
     }
+    __syncthreads();  // every wave's loads are there, and its reads of this token's rows are done
   }
 }
 
@@ -264,10 +300,12 @@ extern "C" int ekv_vha_inv_rope_fp8_quant(const uint16_t* o, int64_t o_tok_strid
   EKV_CHECK(aligned4(out) && aligned4(scale), "misaligned outputs");
   EKV_CHECK(cs_stride >= rope_dim, "cos_sin rows must hold rope_dim entries");
   VhaArgs a{o, o_tok_stride, o_head_stride, mix, positions, cos_sin, cs_stride, num_tokens, aligned_tokens,
-            heads / n_groups, nope_dim, rope_dim / 2, out, reinterpret_cast<uint8_t*>(scale)};
-  const int grid = aligned_tokens < 1024 ? aligned_tokens : 1024;
+            heads / n_groups, nope_dim, rope_dim / 2, out, reinterpret_cast<uint8_t*>(scale), aligned16(out)};
+  const int grid = aligned_tokens < kVhaGrid ? aligned_tokens : kVhaGrid;
+  constexpr int kSmem = static_cast<int>(sizeof(VhaSmem));
   (void)hipFuncSetAttribute(reinterpret_cast<const void*>(vha_inv_rope_quant_kernel),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, kVhaLds);
-  hipLaunchKernelGGL(vha_inv_rope_quant_kernel, dim3(grid), dim3(256), kVhaLds, static_cast<hipStream_t>(stream), a);
+                            hipFuncAttributeMaxDynamicSharedMemorySize, kSmem);
+  hipLaunchKernelGGL(vha_inv_rope_quant_kernel, dim3(grid), dim3(64 * kVhaWaves), kSmem,
+                     static_cast<hipStream_t>(stream), a);
   return ekv_launch_status();
 }
