@@ -3304,7 +3304,15 @@ template <int kWaves, bool kFp4>
 bool plan_fused(int64_t T, int32_t max_len, int64_t pages, int cus, int64_t target_groups, FilterPlan& p) {
   if (T > kCounterRows) return false;
   const void* kernel = reinterpret_cast<const void*>(filter_verify_kernel<kWaves, kFp4>);
-  int64_t groups = std::max<int64_t>(1, std::min<int64_t>((pages + kWaves - 1) / kWaves, (target_groups + T - 1) / T));
+  // At least this many pages a workgroup: fewer than a page a wave leaves waves
+  // without a page to stream, but spreads a small batch's exact scoring, which
+  // is the larger part of it, over more CUs (one sequence of 4096: the step
+  // 68.8 us with 12, 65.5 with 6, 64.5 with 4, 63.6 with 2; of 20000: 65.2,
+  // 63.9, 64.0, 67.8; fp4 keys, whose scoring is cheaper: 42.7, 40.5, 39.4, 39.6
+  // and 37.5, 37.7, 38.8, 43.8).
+  constexpr int kMinPages = std::min(kWaves, kFp4 ? 6 : 4);
+  int64_t groups =
+      std::max<int64_t>(1, std::min<int64_t>((pages + kMinPages - 1) / kMinPages, (target_groups + T - 1) / T));
   for (int attempt = 0; attempt < 4 && groups >= 1; ++attempt) {
     const int per_group = fused_group_pages(max_len, static_cast<int>(groups));
     const int stage = std::max(4, (per_group + 3) & ~3);
