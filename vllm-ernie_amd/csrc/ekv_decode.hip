@@ -692,7 +692,6 @@ __global__ void __launch_bounds__(256) decode_combine_kernel(
   const int wave = kW > 1 ? threadIdx.x >> 6 : 0;
   const int h = kW > 1 ? blockIdx.x : 4 * blockIdx.x + (threadIdx.x >> 6), t = blockIdx.y;
   if (h >= heads) return;
-  const float sk = sinks != nullptr ? sinks[h] * kLog2e : -INFINITY;
   const int2 rs = ws_rows[t];
   const int splits = rs.y;
   if (splits <= 1) return;
@@ -762,6 +761,7 @@ __global__ void __launch_bounds__(256) decode_combine_kernel(
   float den = L;
   float numf = 1.0f;
   if (sinks != nullptr) {
+    const float sk = sinks[h] * kLog2e;
     const float Mp = fmaxf(M, sk);
     if (Mp != -INFINITY) {
       numf = (M == -INFINITY) ? 0.0f : exp2f(M - Mp);
