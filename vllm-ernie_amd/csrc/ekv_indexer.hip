@@ -3033,7 +3033,7 @@ __global__ void __launch_bounds__(kSelThreads) topk_select_kernel(SelectArgs a) 
     const int common = (kmin == kmax) ? 32 : __clz(static_cast<int>(kmin ^ kmax));
     uint32_t mask = common == 0 ? 0u : (common == 32 ? 0xffffffffu : 0xffffffffu << (32 - common));
     uint32_t prefix = kmin & mask;
-    int remaining = k - sure;
+    int remaining = max(1, k - sure);  // (fewer than k are sure unless scores are not finite)
     int top = 32 - common;  // bits [0, top) are still open
     bool first = true;      // the first pass's key range is [kmin, kmax]
     while (top > 0) {
