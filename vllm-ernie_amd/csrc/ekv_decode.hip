@@ -679,9 +679,10 @@ sparse_decode_kernel(DecodeArgs a) {
 // in LDS, each thread finishing two channels.  Bound by memory latency (the
 // partials, 2 KB per split and head, come from other XCDs' writes), so the
 // splits' loads go out together.  Many splits a row: 4 waves (one row of 68
-// splits: 6.7 us, 14.7 with a wave per head); few: a wave per head (32 rows of
-// 8: 8.4 us, 10.4 with 4 waves; 64 of 4: 7.6, 12.7).  Rows finished by their
-// only split are skipped.
+// splits: 6.7 us, 14.7 with a wave per head).  Up to 16: a wave per head (32
+// rows of 8: 8.4 us, 10.4 with 4 waves; 64 of 4: 7.6, 12.7; 27 of 9: the same
+// with the partials in the caches, but a step on a workspace just allocated
+// 431 us against 481-519).  Rows finished by their only split are skipped.
 template <int kW>
 __global__ void __launch_bounds__(256) decode_combine_kernel(
     const float* ws_o, const float* ws_ml, const int2* ws_rows, int32_t heads, const float* sinks,
@@ -860,7 +861,7 @@ extern "C" int ekv_sparse_mla_decode(const uint16_t* q, int64_t q_tok_stride, in
   }
   int rc = ekv_launch_status();
   if (rc) return rc;
-  if (groups > 8 * static_cast<int64_t>(num_tokens))  // more than 8 splits a row
+  if (groups > 16 * static_cast<int64_t>(num_tokens))  // more than 16 splits a row
     hipLaunchKernelGGL(decode_combine_kernel<4>, dim3(heads, num_tokens), dim3(256), 0, s, ws_o, ws_ml, ws_rows, heads,
                        sinks, out, out_tok_stride, out_head_stride, lse, lse_stride);
   else
