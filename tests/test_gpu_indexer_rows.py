@@ -3,8 +3,9 @@ shared-page filter, its per-row bounds and the select of its candidates give
 the same indices as exact scores of every token and the exact select over
 them, both of which test_gpu_indexer holds against the oracle bit for bit.
 Rows of one request (causal lengths), of several with group boundaries inside
-a workgroup's rows, and of mixed requests; unmapped pages, ties, constant rows
-and rows shorter than k."""
+a workgroup's rows, and of mixed requests; unmapped pages, ties, constant rows,
+rows shorter than k, and scores that are infinite (fp32 overflow of
+finite operands; more and fewer than k of them, and all) or NaN."""
 
 import numpy as np
 import pytest
@@ -29,15 +30,23 @@ def _case(dev, T, n_seqs, order, max_len, kind, seed):
         k = k[torch.randint(0, 30, (n,), device=dev, generator=g)]
     elif kind == "constant":
         k = k[:1].expand(n, 128)
+    elif kind == "overflow":  # of every 7 keys one scores beyond fp32 (about half of them +inf, half -inf)
+        k[::7] *= 1e36
+    elif kind == "all inf":
+        k = k.abs() * 1e36
     ops.indexer_k_insert(k.bfloat16().contiguous(), torch.arange(n, device=dev), kcache)
     if kind == "unmapped":
         bt[:, 1] = -1
         bt[-1, -1] = n_seqs * pages + 7
+    if kind == "nan":
+        kcache[:, 64 * 128:].view(torch.float32)[:, ::9] = float("nan")
     req = np.sort(rng.integers(0, n_seqs, T)) if order == "runs" else rng.integers(0, n_seqs, T)
     req = req.astype(np.int32)
     lengths = np.minimum(max_len, 1 + np.arange(T) % (max_len + 40)).astype(np.int32)
     q = torch.randn(T, 64, 128, device=dev, generator=g).bfloat16()
     w = torch.randn(T, 64, device=dev, generator=g).bfloat16()
+    if kind == "all inf":
+        q, w = q.abs(), w.abs()
     return (*ops.indexer_q_quant(q, w), kcache, to_dev(bt, dev), to_dev(req, dev), to_dev(lengths, dev))
 
 
@@ -47,6 +56,10 @@ def _case(dev, T, n_seqs, order, max_len, kind, seed):
     (1031, 5, "mixed", 640, 64, "normal"),
     (1040, 1, "runs", 2500, 2048, "unmapped"),
     (1032, 2, "runs", 700, 500, "constant"),
+    (1030, 2, "runs", 900, 40, "overflow"),
+    (1030, 2, "runs", 900, 200, "overflow"),
+    (1026, 1, "runs", 500, 100, "all inf"),
+    (1026, 3, "mixed", 600, 100, "nan"),
 ])
 def test_many_rows_topk_matches_exact_scores(dev, T, n_seqs, order, max_len, k, kind):
     from ernie_kv import ops
@@ -54,6 +67,8 @@ def test_many_rows_topk_matches_exact_scores(dev, T, n_seqs, order, max_len, k, 
     q8, w, dig, kcache, bt, req, lengths = _case(dev, T, n_seqs, order, max_len, kind, T + max_len)
     scores = torch.full((T, max_len), float("nan"), device=dev)
     ops.indexer_score(dig, w, kcache, bt, req, lengths, max_len, scores)
+    n_inf = int((scores == float("inf")).sum(1).max())
+    assert n_inf == max_len if kind == "all inf" else 40 < n_inf < 200 if kind == "overflow" else n_inf == 0
     ref = torch.empty((T, k), dtype=torch.int32, device=dev)
     ops.topk_select(scores, lengths, k, ref)
     got = torch.empty((T, k), dtype=torch.int32, device=dev)

@@ -880,8 +880,15 @@ __device__ __forceinline__ float page_sums(const float (&acc)[4]) {
   return f(c[0]) + f(c[1]);
 }
 
-// The two bounds of a token as one word.
+// The two bounds of a token as one word.  With both e and its factor before
+// the key scale (RowOps::eb) at most 2^100 every sum of the approximate and of
+// the exact score stays below 2^115, so the bound holds; otherwise (sums that
+// may overflow, operands that are not finite) the word bounds nothing: U is
+// the largest key, L the smallest, and the token is scored.  L <= U as keys in
+// either case.
+constexpr float kBoundMax = 0x1p100f;
 __device__ __forceinline__ uint32_t bound_word(float sc, float e) {
+  if (!(fabsf(sc) <= 0x1p120f && e >= 0.0f && e <= kBoundMax)) return 0x7fffffffu;
   const uint32_t up = bf16_round_up(sc + e);
   const uint32_t dn = bf16_round_up(-(sc - e)) ^ 0x8000u;
   return (up << 16) | dn;
@@ -890,7 +897,7 @@ __device__ __forceinline__ uint32_t bound_word(float sc, float e) {
 struct RowOps {
   i32x8 qa[kRowsWave][4];
   float wv[kRowsWave][4][4];
-  float eb[kRowsWave];
+  float eb[kRowsWave];  // inf when larger than kBoundMax
 };
 
 // Adds a block's 16 tokens (kv) to the wave's rows' sums.
@@ -951,7 +958,7 @@ filter_rows_kernel(FilterArgs a, uint32_t* bounds) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) op.wv[r][hb][i] = f.wv[hb][i];
     }
-    op.eb[r] = f.eb[0];
+    op.eb[r] = f.eb[0] <= kBoundMax ? f.eb[0] : INFINITY;
   }
   auto word = [&](int r, const float (&acc)[4], float scale) -> uint32_t {
     return bound_word(page_sums(acc) * scale, scale * op.eb[r]);
@@ -1179,12 +1186,13 @@ struct VerifyArgs {
   const uint32_t* kin;       // kRows: [T]
 };
 
+constexpr uint32_t kSureMark = 0x80000000u;  // bit of a listed token that is selected whatever its score
 constexpr int kVerifyChunks = 4;  // chunks per verify workgroup
 constexpr int kVerifyPages = kVerifyChunks * kChunk / kPageTokens;
 
 // kRows: the bounds are filter_rows_kernel's words, and a candidate whose
-// lower bound is above kin is selected in any case: it is listed with score
-// +inf instead of being scored (about two thirds of a row's candidates).
+// lower bound is above kin is selected in any case: it is listed unscored,
+// its index marked with kSureMark (about two thirds of a row's candidates).
 template <bool kFp4, bool kRows = false>
 __global__ void __launch_bounds__(256) verify_kernel(VerifyArgs a) {
   __shared__ uint32_t s_table[256];  // fp8: digit table; fp4: q scale words
@@ -1283,8 +1291,7 @@ __global__ void __launch_bounds__(256) verify_kernel(VerifyArgs a) {
         if (flags & (1u << j)) {
           if (sure & (1u << j)) {
             const int64_t dst = row + static_cast<int64_t>(c) * kChunk + slot;
-            a.cand_score[dst] = INFINITY;
-            a.cand_idx[dst] = chunk0 + start + j;
+            a.cand_idx[dst] = static_cast<int32_t>(static_cast<uint32_t>(chunk0 + start + j) | kSureMark);
           } else {
             s_list[pos] = static_cast<int16_t>(chunk0 + start + j - tok0);
             s_meta[pos] = static_cast<int16_t>((cc << 11) | slot);
@@ -2796,13 +2803,13 @@ struct SelectArgs {
   const int32_t* cand_idx;
   const int32_t* cand_count; // [T, chunks]
   int32_t chunks;
-  float* stage_score;        // chunk mode spill: [T, max_len]
+  uint32_t* stage_key;       // chunk mode spill: [T, max_len]
   int32_t* stage_idx;
   int32_t* out;              // [T, out_stride]
   int64_t out_stride;
   int32_t k;
   int32_t max_len;
-  int32_t sure;              // chunk mode: a score of +inf is a token selected in any case
+  int32_t sure;              // chunk mode: listed tokens may carry kSureMark
   int32_t seg_groups;        // chunk mode: 0 = lists of kChunk-token chunks, else of
                              // filter_verify_kernel segments (`seg_groups` per row)
   // Optional merged output (merge_swa_topk of the result): [T, merged_stride]
@@ -2899,13 +2906,16 @@ __global__ void __launch_bounds__(kSelThreads) topk_select_kernel(SelectArgs a) 
 
   // gather the elements; lo / hi track the range of the keys put in LDS
   uint32_t lo = 0xffffffffu, hi = 0u;
-  // The key of sure tokens (0: none): they are above the threshold and take no
-  // part in the passes that look for it.
-  const uint32_t sure_key = a.sure ? score_key(INFINITY) : 0u;
+  // The key of marked tokens (0: none): they are above the threshold and take no
+  // part in the passes that look for it.  No scored token has it (a NaN that
+  // would is taken one lower).  Fewer than k tokens are marked: each has fewer
+  // than k tokens whose upper bound reaches its lower bound.
+  const uint32_t sure_key = a.sure ? 0xffffffffu : 0u;
   int sure = 0;  // this thread's
   int n;
-  const float* gsc = nullptr;     // global scores (implicit mode or spilled lists)
-  const int32_t* gidx = nullptr;  // global indices (spilled lists); null = implicit
+  const float* gsc = nullptr;      // implicit mode: global scores
+  const uint32_t* gkey = nullptr;  // spilled lists: global keys and indices
+  const int32_t* gidx = nullptr;
   bool in_lds;
   if (a.cand_count == nullptr) {
     n = max(0, min(a.lengths[t], a.max_len));
@@ -2939,7 +2949,7 @@ __global__ void __launch_bounds__(kSelThreads) topk_select_kernel(SelectArgs a) 
     const int64_t seg = a.seg_groups > 0
                             ? kPageTokens * fused_group_pages(max(0, min(a.lengths[t], a.max_len)), a.seg_groups)
                             : kChunk;  // tokens per list slice
-    float* st_sc = a.stage_score + row;
+    uint32_t* st_key = a.stage_key + row;
     int32_t* st_ix = a.stage_idx + row;
     // Position p of the concatenation lies in list c = the last with
     // off[c] <= p (binary search; empty lists are skipped by construction).
@@ -2973,24 +2983,31 @@ __global__ void __launch_bounds__(kSelThreads) topk_select_kernel(SelectArgs a) 
       for (int q = 0; q < kGather; ++q) {
         const int p = p0 + q * kSelThreads + tid;
         if (p >= n) continue;
-        const uint32_t key = score_key(sv[q] + 0.0f);
-        if (sure_key != 0u && key == sure_key) ++sure;
+        uint32_t key = score_key(sv[q] + 0.0f);
+        int32_t ix = iv[q];
+        bool marked = false;
+        if (sure_key != 0u) {
+          marked = ix < 0;
+          key = marked ? sure_key : min(key, sure_key - 1u);
+          ix = static_cast<int32_t>(static_cast<uint32_t>(ix) & ~kSureMark);
+        }
+        if (marked) ++sure;
         else if (in_lds) {
           lo = min(lo, key);
           hi = max(hi, key);
         }
         if (in_lds) {
           s_key[p] = key;
-          s_idx[p] = iv[q];
+          s_idx[p] = ix;
         } else {
-          st_sc[p] = sv[q];
-          st_ix[p] = iv[q];
+          st_key[p] = key;
+          st_ix[p] = ix;
         }
       }
     }
     if (!in_lds) {
       __threadfence_block();
-      gsc = st_sc;
+      gkey = st_key;
       gidx = st_ix;
     }
   }
@@ -3011,7 +3028,9 @@ __global__ void __launch_bounds__(kSelThreads) topk_select_kernel(SelectArgs a) 
     for (int w = 0; w < kSelThreads / 64; ++w) sure += sm.wave[w];
     __syncthreads();
   }
-  auto key_at = [&](int i) -> uint32_t { return in_lds ? s_key[i] : score_key(gsc[i] + 0.0f); };
+  auto key_at = [&](int i) -> uint32_t {
+    return in_lds ? s_key[i] : (gkey ? gkey[i] : score_key(gsc[i] + 0.0f));
+  };
   auto idx_at = [&](int i) -> int32_t { return in_lds ? s_idx[i] : (gidx ? gidx[i] : i); };
 
   uint32_t kstar = 0;
@@ -3033,7 +3052,7 @@ __global__ void __launch_bounds__(kSelThreads) topk_select_kernel(SelectArgs a) 
     const int common = (kmin == kmax) ? 32 : __clz(static_cast<int>(kmin ^ kmax));
     uint32_t mask = common == 0 ? 0u : (common == 32 ? 0xffffffffu : 0xffffffffu << (32 - common));
     uint32_t prefix = kmin & mask;
-    int remaining = max(1, k - sure);  // (fewer than k are sure unless scores are not finite)
+    int remaining = k - sure;  // at least 1; the tokens not marked number more (n > k)
     int top = 32 - common;  // bits [0, top) are still open
     bool first = true;      // the first pass's key range is [kmin, kmax]
     while (top > 0) {
@@ -3228,7 +3247,7 @@ int64_t count_slots(int64_t T, int32_t max_len) { return T * num_chunks(max_len)
 // workspace: timeouts u32 [4] (cumulative), padded to 256 B | fused-path
 //            counters u32 [kCounterRows, kCounterRow] (kept zero between
 //            calls) | upper u16 [T,L] (4 B per entry reserved) |
-//            cand_score f32 [T,L] | cand_idx i32 [T,L] | stage_score f32 [T,L] |
+//            cand_score f32 [T,L] | cand_idx i32 [T,L] | stage_key u32 [T,L] |
 //            stage_idx i32 [T,L] | hist u32 [T,4096] | arrive u32 [T] |
 //            kbound u32 [T] (the unfused path's, cleared per call) |
 //            counts i32 [count_slots]
@@ -3239,7 +3258,7 @@ struct TopkWorkspace {
   uint16_t* upper;
   float* cand_score;
   int32_t* cand_idx;
-  float* stage_score;
+  uint32_t* stage_key;
   int32_t* stage_idx;
   uint32_t* hist;
   uint32_t* arrive;
@@ -3256,8 +3275,8 @@ TopkWorkspace carve(void* workspace, int64_t T, int64_t L) {
   w.upper = reinterpret_cast<uint16_t*>(base + kCounterBytes);
   w.cand_score = reinterpret_cast<float*>(base + kCounterBytes + T * L * 4);
   w.cand_idx = reinterpret_cast<int32_t*>(w.cand_score + T * L);
-  w.stage_score = reinterpret_cast<float*>(w.cand_idx + T * L);
-  w.stage_idx = reinterpret_cast<int32_t*>(w.stage_score + T * L);
+  w.stage_key = reinterpret_cast<uint32_t*>(w.cand_idx + T * L);
+  w.stage_idx = reinterpret_cast<int32_t*>(w.stage_key + T * L);
   w.hist = reinterpret_cast<uint32_t*>(w.stage_idx + T * L);
   w.arrive = w.hist + T * kHistBins;
   w.kbound = w.arrive + T;
@@ -3573,7 +3592,7 @@ int run_select(const TopkQuery& q, const uint8_t* kcache, int64_t page_stride, i
     }
   }
   SelectArgs sel{nullptr, 0, lengths, ws.cand_score, ws.cand_idx, ws.counts, plan.fused ? plan.groups : chunks,
-                 ws.stage_score, ws.stage_idx, topk_out, out_stride, k, static_cast<int32_t>(L),
+                 ws.stage_key, ws.stage_idx, topk_out, out_stride, k, static_cast<int32_t>(L),
                  plan.rows ? 1 : 0, plan.fused ? plan.groups : 0, merged_out, merged_stride, merged_width, positions, window,
                  merged_slots ? block_table : nullptr, bt_stride, req_ids, num_pages};
   launch_select(sel, num_tokens, s);
