@@ -31,9 +31,9 @@ def _case(dev, T, n_seqs, order, max_len, kind, seed):
     elif kind == "constant":
         k = k[:1].expand(n, 128)
     elif kind == "overflow":  # of every 7 keys one scores beyond fp32 (about half of them +inf, half -inf)
-        k[::7] *= 1e36
+        k[::7] *= 1e37
     elif kind == "all inf":
-        k = k.abs() * 1e36
+        k = k.abs() * 1e37
     ops.indexer_k_insert(k.bfloat16().contiguous(), torch.arange(n, device=dev), kcache)
     if kind == "unmapped":
         bt[:, 1] = -1
@@ -45,6 +45,8 @@ def _case(dev, T, n_seqs, order, max_len, kind, seed):
     lengths = np.minimum(max_len, 1 + np.arange(T) % (max_len + 40)).astype(np.int32)
     q = torch.randn(T, 64, 128, device=dev, generator=g).bfloat16()
     w = torch.randn(T, 64, device=dev, generator=g).bfloat16()
+    if kind in ("overflow", "all inf"):
+        w = w * 1024
     if kind == "all inf":
         q, w = q.abs(), w.abs()
     return (*ops.indexer_q_quant(q, w), kcache, to_dev(bt, dev), to_dev(req, dev), to_dev(lengths, dev))
