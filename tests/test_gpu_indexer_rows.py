@@ -76,3 +76,21 @@ def test_many_rows_topk_matches_exact_scores(dev, T, n_seqs, order, max_len, k, 
     got = torch.empty((T, k), dtype=torch.int32, device=dev)
     ops.indexer_topk(q8, dig, w, kcache, bt, req, lengths, max_len, got)
     assert torch.equal(got, ref)
+
+@pytest.mark.parametrize("order", ["runs", "mixed"])
+def test_many_rows_select_of_fewer_than_filtered(dev, order):
+    """The two stages with a select of fewer tokens than the filter's k: also
+    for rows between the two, which the filter left alone."""
+    from ernie_kv import ops
+
+    T, max_len, k = 1027, 900, 48
+    q8, w, dig, kcache, bt, req, lengths = _case(dev, T, 3, order, max_len, "normal", 5)
+    scores = torch.full((T, max_len), float("nan"), device=dev)
+    ops.indexer_score(dig, w, kcache, bt, req, lengths, max_len, scores)
+    ref = torch.empty((T, k), dtype=torch.int32, device=dev)
+    ops.topk_select(scores, lengths, k, ref)
+    ws = ops.indexer_topk_workspace(T, max_len, dev)
+    got = torch.empty((T, k), dtype=torch.int32, device=dev)
+    ops.indexer_filter(q8, dig, w, kcache, bt, req, lengths, max_len, ws, k=300)
+    ops.indexer_select(dig, w, kcache, bt, req, lengths, max_len, got, ws)
+    assert torch.equal(got, ref)

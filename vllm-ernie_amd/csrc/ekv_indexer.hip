@@ -1072,17 +1072,27 @@ filter_rows_kernel(FilterArgs a, uint32_t* bounds) {
 // high half, as a score key) of the k-th largest L -- a token whose U is below
 // it has k tokens above it -- and kin[t] of the k-th largest U: fewer than k
 // tokens can reach a token whose L is above it, so it is selected whatever its
-// exact score.  One workgroup per row: the bounds' high 12 key bits, then the
-// low 4 of the two threshold bins.
+// exact score (by a select of k or more; kfilter[t] keeps k).  A row of at
+// most k tokens has no bounds: every token is a candidate, none vouched for.
+// One workgroup per row: the bounds' high 12 key bits, then the low 4 of the
+// two threshold bins.
 __global__ void __launch_bounds__(512) row_bounds_kernel(const uint32_t* bounds, const int32_t* lengths,
-                                                         int32_t max_len, int32_t k, uint32_t* kbound, uint32_t* kin) {
+                                                         int32_t max_len, int32_t k, uint32_t* kbound, uint32_t* kin,
+                                                         uint32_t* kfilter) {
   __shared__ uint32_t s_hist[2][kHistBins];  // [0] of U, [1] of L
   __shared__ uint32_t s_low[2][16];
   __shared__ int s_wave[8];
   __shared__ int s_res[2];
   const int tid = threadIdx.x, t = blockIdx.x;
   const int n = min(lengths[t], max_len);
-  if (n <= k) return;  // unused: every token is selected
+  if (tid == 0) kfilter[t] = static_cast<uint32_t>(k);
+  if (n <= k) {
+    if (tid == 0) {
+      kbound[t] = 0u;
+      kin[t] = 0xffffu;
+    }
+    return;
+  }
   for (int i = tid; i < 2 * kHistBins; i += 512) s_hist[0][i] = 0;
   if (tid < 32) s_low[0][tid] = 0;
   __syncthreads();
@@ -1184,6 +1194,7 @@ struct VerifyArgs {
   const int32_t* q_scales;   // fp4 keys: [T, 64]
   const uint32_t* bounds;    // kRows: [T, max_len] words of filter_rows_kernel (upper unused)
   const uint32_t* kin;       // kRows: [T]
+  const uint32_t* kfilter;   // kRows: [T], the k that kin holds for
 };
 
 constexpr uint32_t kSureMark = 0x80000000u;  // bit of a listed token that is selected whatever its score
@@ -1249,7 +1260,9 @@ __global__ void __launch_bounds__(256) verify_kernel(VerifyArgs a) {
   const int start = tid * kPer;
   int total = 0;
   if constexpr (kRows) {
-    const uint32_t kb16 = kbound >> 16, kin = a.kin[t];
+    const uint32_t kb16 = kbound >> 16;
+    // (a smaller k than the filter's: no token is vouched for)
+    const uint32_t kin = static_cast<uint32_t>(a.k) >= a.kfilter[t] ? a.kin[t] : 0xffffu;
     uint32_t wd[kVerifyChunks][kPer];
 #pragma unroll
     for (int cc = 0; cc < kVerifyChunks; ++cc) {
@@ -3251,6 +3264,8 @@ int64_t count_slots(int64_t T, int32_t max_len) { return T * num_chunks(max_len)
 //            stage_idx i32 [T,L] | hist u32 [T,4096] | arrive u32 [T] |
 //            kbound u32 [T] (the unfused path's, cleared per call) |
 //            counts i32 [count_slots]
+// The many-row path keeps bound words u32 [T,L] at `upper`, kfilter [T] at
+// `hist` and kin [T] at `arrive`; it writes all it reads, so clears none.
 // The front (timeouts and counters) sits at the same offsets for every
 // (T, L), so one zero-filled allocation serves calls of any shape.
 struct TopkWorkspace {
@@ -3545,7 +3560,7 @@ int run_filter(const TopkQuery& q, const uint8_t* kcache, int64_t page_stride, i
     hipLaunchKernelGGL(filter_rows_kernel, dim3(static_cast<unsigned>(8 * ((row_groups + 7) / 8) * plan.groups)),
                        dim3(64 * kRowsWaves), 0, s, f, bounds);
     hipLaunchKernelGGL(row_bounds_kernel, dim3(num_tokens), dim3(512), 0, s, bounds, lengths, max_len, k, ws.kbound,
-                       ws.arrive);
+                       ws.arrive, ws.hist);
   } else if (max_len > 0) {
     const int64_t nz = T * kHistBins + 2 * T;  // this call's hist, arrive, kbound
     const int64_t zero_blocks = (nz + 255) / 256;
@@ -3583,7 +3598,7 @@ int run_select(const TopkQuery& q, const uint8_t* kcache, int64_t page_stride, i
   if (!plan.fused) {
     VerifyArgs v{q.q_digits, q.w, kcache, page_stride, num_pages, block_table, bt_stride, req_ids, lengths,
                  max_len, k, ws.upper, ws.kbound, ws.cand_score, ws.cand_idx, ws.counts, chunks,
-                 kFp4 ? q.q : nullptr, q.q_scales, reinterpret_cast<const uint32_t*>(ws.upper), ws.arrive};
+                 kFp4 ? q.q : nullptr, q.q_scales, reinterpret_cast<const uint32_t*>(ws.upper), ws.arrive, ws.hist};
     const dim3 grid((chunks + kVerifyChunks - 1) / kVerifyChunks, num_tokens);
     if (plan.rows && max_len > 0) {
       if constexpr (!kFp4) hipLaunchKernelGGL((verify_kernel<false, true>), grid, dim3(256), 0, s, v);
