@@ -94,3 +94,20 @@ def test_many_rows_select_of_fewer_than_filtered(dev, order):
     ops.indexer_filter(q8, dig, w, kcache, bt, req, lengths, max_len, ws, k=300)
     ops.indexer_select(dig, w, kcache, bt, req, lengths, max_len, got, ws)
     assert torch.equal(got, ref)
+
+@pytest.mark.parametrize("T", [3, 1027])
+def test_topk_of_zero_max_len(dev, T):
+    """max_len 0 admits no token, whatever the rows' lengths say: all -1, in
+    one call and in two stages."""
+    from ernie_kv import ops
+
+    q8, w, dig, kcache, bt, req, lengths = _case(dev, T, 2, "runs", 130, "normal", 6)
+    ws = ops.indexer_topk_workspace(T, 0, dev)
+    for staged in (False, True):
+        got = torch.zeros((T, 16), dtype=torch.int32, device=dev)
+        if staged:
+            ops.indexer_filter(q8, dig, w, kcache, bt, req, lengths, 0, ws, k=16)
+            ops.indexer_select(dig, w, kcache, bt, req, lengths, 0, got, ws)
+        else:
+            ops.indexer_topk(q8, dig, w, kcache, bt, req, lengths, 0, got, ws)
+        assert (got == -1).all()

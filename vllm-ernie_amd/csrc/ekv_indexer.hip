@@ -3607,7 +3607,7 @@ int run_select(const TopkQuery& q, const uint8_t* kcache, int64_t page_stride, i
     }
   }
   SelectArgs sel{nullptr, 0, lengths, ws.cand_score, ws.cand_idx, ws.counts, plan.fused ? plan.groups : chunks,
-                 ws.stage_key, ws.stage_idx, topk_out, out_stride, k, static_cast<int32_t>(L),
+                 ws.stage_key, ws.stage_idx, topk_out, out_stride, k, max_len,
                  plan.rows ? 1 : 0, plan.fused ? plan.groups : 0, merged_out, merged_stride, merged_width, positions, window,
                  merged_slots ? block_table : nullptr, bt_stride, req_ids, num_pages};
   launch_select(sel, num_tokens, s);
