@@ -1222,17 +1222,9 @@ __global__ void __launch_bounds__(256) verify_kernel(VerifyArgs a) {
   const int64_t row = static_cast<int64_t>(t) * a.max_len;
   const int c_begin = blockIdx.x * kVerifyChunks;
   int32_t* counts = a.cand_count + static_cast<int64_t>(t) * a.chunks;
+  if (n <= a.k) return;  // every token is selected: the select reads no lists
   if (c_begin * kChunk >= n) {  // every chunk past the row's end: empty lists
     if (tid < kVerifyChunks && c_begin + tid < a.chunks) counts[c_begin + tid] = 0;
-    return;
-  }
-  if (n <= a.k) {  // every token is selected: list them, no scores needed
-    for (int c = c_begin; c < min(c_begin + kVerifyChunks, a.chunks); ++c) {
-      const int chunk0 = c * kChunk;
-      const int len = max(0, min(kChunk, n - chunk0));
-      for (int i = tid; i < len; i += 256) a.cand_idx[row + chunk0 + i] = chunk0 + i;
-      if (tid == 0) counts[c] = len;
-    }
     return;
   }
   const int lane = tid & 63, wave = tid >> 6;
