@@ -888,10 +888,10 @@ __device__ __forceinline__ float page_sums(const float (&acc)[4]) {
 // either case.
 constexpr float kBoundMax = 0x1p100f;
 __device__ __forceinline__ uint32_t bound_word(float sc, float e) {
-  if (!(fabsf(sc) <= 0x1p120f && e >= 0.0f && e <= kBoundMax)) return 0x7fffffffu;
+  const bool holds = (fabsf(sc) <= 0x1p120f) & (e >= 0.0f) & (e <= kBoundMax);
   const uint32_t up = bf16_round_up(sc + e);
   const uint32_t dn = bf16_round_up(-(sc - e)) ^ 0x8000u;
-  return (up << 16) | dn;
+  return holds ? (up << 16) | dn : 0x7fffffffu;
 }
 
 struct RowOps {
