@@ -58,6 +58,21 @@ def test_rows_dispatch_edges(dev, T, heads, width):
     _run(dev, rng, 576, heads, np.maximum(idx, -1), lengths)
 
 
+@pytest.mark.parametrize("T,heads,width,dim,bf16", [
+    (128, 64, 192, 576, True), (129, 64, 192, 576, True), (96, 48, 1500, 512, True), (104, 48, 1500, 512, True),
+    (192, 32, 769, 512, True), (257, 16, 769, 576, True), (384, 16, 769, 512, True), (7, 48, 256, 576, False),
+    (8, 48, 256, 576, False), (120, 48, 1152, 576, False), (128, 48, 1152, 576, False)])
+def test_dispatch_lines(dev, T, heads, width, dim, bf16):
+    """Both sides of the lines between the two kernels that depend on the cache
+    type, the heads and the few-row kernel's workgroups.  Most rows are short, a
+    few full."""
+    rng = np.random.default_rng(T + heads + width)
+    idx = rng.integers(-100, 40 * 64, (T, width)).astype(np.int32)
+    lengths = rng.integers(0, 40, T).astype(np.int32)
+    lengths[::50] = width
+    _run(dev, rng, dim, heads, np.maximum(idx, -1), lengths, bf16)
+
+
 @pytest.mark.parametrize("factor", [8.0, 96.0])
 def test_rows_reference_moves(dev, factor):
     """Later steps hold rows `factor` times larger: scores a few tens, or more

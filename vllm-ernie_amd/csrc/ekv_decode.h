@@ -81,8 +81,9 @@ __device__ __forceinline__ i16x4 lds_read_tr16(const uint8_t* p) {
 }
 
 // The whole-row kernel (ekv_decode_rows.hip): whether a call of num_tokens rows
-// of `width` entries takes it, and its launch.
-bool decode_rows_takes(int32_t num_tokens, int32_t heads, int32_t width);
+// of `width` entries takes it (the few-row kernel would launch split_groups
+// workgroups), and its launch.
+bool decode_rows_takes(int32_t num_tokens, int32_t heads, int32_t width, bool cache_bf16, int64_t split_groups);
 int launch_decode_rows(const DecodeArgs& a, int32_t dim, bool cache_bf16, hipStream_t s);
 
 }  // namespace ekv

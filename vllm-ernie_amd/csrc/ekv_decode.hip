@@ -850,7 +850,8 @@ extern "C" int ekv_sparse_mla_decode(const uint16_t* q, int64_t q_tok_stride, in
                static_cast<int32_t>(groups), ws_o, ws_ml, ws_rows, sinks, out, out_tok_stride, out_head_stride,
                lse, lse_stride};
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (decode_rows_takes(num_tokens, heads, width)) return launch_decode_rows(a, dim, cache_bf16 != 0, s);
+  if (decode_rows_takes(num_tokens, heads, width, cache_bf16 != 0, groups))
+    return launch_decode_rows(a, dim, cache_bf16 != 0, s);
   const dim3 grid(static_cast<uint32_t>(groups));
   if (dim == 576) {
     if (cache_bf16) launch_decode<576, true>(a, grid, s);

@@ -2,9 +2,9 @@
 // ekv_decode.hip: gathered latent rows with the per-head attention sink in the
 // softmax denominator.
 //
-// Workgroup = (query row t, block of 32 heads), 4
-// waves, two workgroups a CU.  The row's valid entries go through in steps of
-// 32 cache rows; wave w:
+// Workgroup = (query row t, block of 32 heads), 4 waves, two workgroups a CU
+// (bf16 rows: one).  The row's valid entries go through in steps of 32 cache
+// rows; wave w:
 //   * scores: S^T = K Q^T of the 32 heads and rows over the 16-dim blocks 4 ks +
 //     w (v_mfma_f32_32x32x16_bf16, A = the rows from LDS, fp8 converted exactly
 //     to bf16, B = its part of q held in registers); the four waves' sums meet
@@ -613,23 +613,47 @@ void launch(const DecodeArgs& a, hipStream_t s) {
 
 // The line between this kernel (a whole row a workgroup: about 9 us + 1.35 us
 // per 32 entries, no partials) and the few-row one (rows split over the CUs,
-// then a combine), measured at 1..2048 rows of full index rows, 64 / 16 heads:
-//   * from 192 rows on no splitting is needed to fill the CUs (2176 entries:
-//     192 rows 133 us here, 165 there; 256: 137, 216);
-//   * short rows: the combine costs more than the splits give (64 heads, 256
-//     entries: 1 row 19, 21, 64 rows 20, 29; 384: 16 rows 25, 27; 16 heads, 160
-//     entries: 14, 16);
-//   * 33..64 heads, 96..128 rows: two workgroups of a row fill the CUs (2176
-//     entries, 128 rows: 103, 114), and up to 191 rows while the rows are short
-//     enough that running two a CU pays (1152 of which 700 valid, 160 rows: 66,
-//     86; but 2176: 133, 118).
+// then a combine), measured at 1..640 rows of full index rows of 33..2176
+// entries, 16 / 32 / 48 / 64 heads, both widths and cache types.  Ratios are
+// the few-row kernel's time over this one's.
+//   * fp8 caches, two workgroups a CU.  From 192 rows on no splitting is needed
+//     to fill the CUs (64 heads, 2176 entries: 192 rows 1.30, 256: 1.68; the
+//     least from there on 1.01, 48 heads).
+//   * Short rows: the combine costs more than the splits give (64 heads, 256
+//     entries: 1 row 1.11, 64 rows 1.63; 384: 8 rows 0.99, 16 rows 1.23; 48
+//     heads, 2 rows: 192 entries 1.06, 256 0.96; 32 heads, 8 rows: 192 1.13, 256
+//     0.97).
+//   * 33..64 heads, 96..128 rows: two workgroups of a row fill the CUs (64 heads,
+//     128 rows: 2176 entries 1.17, 768 1.12).  The few-row kernel runs its
+//     workgroups at once while they number at most 256, and is the faster one
+//     for long rows up to there (48 heads, 1152 entries: 120 rows 0.94, 128 rows
+//     1.56).  Up to 191 rows while running two a CU pays (64 heads: 160 rows of
+//     1152 1.32, of 2176 0.96).
+//   * bf16 caches: the row images leave room for one workgroup a CU, so rows
+//     above 32 heads, two workgroups each, fill the CUs once at 128 rows (64
+//     heads, 192 entries: 128 rows 1.64, 136 rows 0.82; 2048 rows of 2176 0.83)
+//     and the gain per row is smaller (64 heads, 8 rows: 192 entries 1.20, 320
+//     1.00; 48 heads, 2 rows: 192 0.99, 256 0.89, 104 rows: 512 1.04, 1800
+//     1.24, 2176 0.92).  Up to 32 heads: from 192 rows on, but not where a
+//     second round of long rows is mostly empty (32 heads, 288 rows: 768
+//     entries 1.04, 2176 0.87; 384 rows of 2176 1.08).
 // Rows past what the LDS holds slots for take the few-row kernel.
-bool decode_rows_takes(int32_t num_tokens, int32_t heads, int32_t width) {
+bool decode_rows_takes(int32_t num_tokens, int32_t heads, int32_t width, bool cache_bf16, int64_t split_groups) {
   if (width > decode_rows::kMaxEntries || num_tokens >= (1 << 28)) return false;
+  if (heads <= 32) {
+    if (num_tokens < 192) return width <= 192;
+    return !cache_bf16 || num_tokens <= 256 || num_tokens >= 384 || width <= 768;
+  }
+  const bool split_rounds = split_groups > 256;  // the few-row kernel's workgroups do not all run at once
+  if (cache_bf16) {
+    if (num_tokens > 128) return false;
+    return width <= 192 || (width <= 320 && num_tokens >= 16) ||
+           (num_tokens >= 96 && (width <= 512 || (split_rounds && width <= 1800)));
+  }
   if (num_tokens >= 192) return true;
-  if (heads <= 32) return width <= 192;
-  return width <= 256 || (width <= 384 && num_tokens >= 16) ||
-         (num_tokens >= 96 && (num_tokens <= 128 || width <= 1152));
+  if (num_tokens > 128) return width <= 1152;
+  return width <= (heads > 48 || num_tokens >= 8 ? 256 : 192) || (width <= 384 && num_tokens >= 16) ||
+         (num_tokens >= 96 && (width <= 768 || split_rounds));
 }
 
 int launch_decode_rows(const DecodeArgs& a, int32_t dim, bool cache_bf16, hipStream_t s) {
