@@ -3,7 +3,7 @@ shared-page filter, its per-row bounds and the select of its candidates give
 the same indices as exact scores of every token and the exact select over
 them, both of which test_gpu_indexer holds against the oracle bit for bit.
 Rows of one request (causal lengths), of several with group boundaries inside
-a workgroup's rows, and of mixed requests; unmapped pages, ties, constant rows,
+a workgroup's rows, of mixed requests and of two or three draft rows; unmapped pages, ties, constant rows,
 rows shorter than k, and scores that are infinite (fp32 overflow of
 finite operands; more and fewer than k of them, and all) or NaN."""
 
@@ -40,7 +40,10 @@ def _case(dev, T, n_seqs, order, max_len, kind, seed):
         bt[-1, -1] = n_seqs * pages + 7
     if kind == "nan":
         kcache[:, 64 * 128:].view(torch.float32)[:, ::9] = float("nan")
-    req = np.sort(rng.integers(0, n_seqs, T)) if order == "runs" else rng.integers(0, n_seqs, T)
+    if order.isdigit():  # that many draft rows a request
+        req = np.arange(T) // int(order)
+    else:
+        req = np.sort(rng.integers(0, n_seqs, T)) if order == "runs" else rng.integers(0, n_seqs, T)
     req = req.astype(np.int32)
     lengths = np.minimum(max_len, 1 + np.arange(T) % (max_len + 40)).astype(np.int32)
     q = torch.randn(T, 64, 128, device=dev, generator=g).bfloat16()
@@ -62,6 +65,8 @@ def _case(dev, T, n_seqs, order, max_len, kind, seed):
     (1030, 2, "runs", 900, 200, "overflow"),
     (1026, 1, "runs", 500, 100, "all inf"),
     (1026, 3, "mixed", 600, 100, "nan"),
+    (1030, 515, "2", 700, 100, "unmapped"),
+    (1027, 343, "3", 400, 64, "ties"),
 ])
 def test_many_rows_topk_matches_exact_scores(dev, T, n_seqs, order, max_len, k, kind):
     from ernie_kv import ops
@@ -76,6 +81,7 @@ def test_many_rows_topk_matches_exact_scores(dev, T, n_seqs, order, max_len, k, 
     got = torch.empty((T, k), dtype=torch.int32, device=dev)
     ops.indexer_topk(q8, dig, w, kcache, bt, req, lengths, max_len, got)
     assert torch.equal(got, ref)
+
 
 @pytest.mark.parametrize("order", ["runs", "mixed"])
 def test_many_rows_select_of_fewer_than_filtered(dev, order):
@@ -94,6 +100,7 @@ def test_many_rows_select_of_fewer_than_filtered(dev, order):
     ops.indexer_filter(q8, dig, w, kcache, bt, req, lengths, max_len, ws, k=300)
     ops.indexer_select(dig, w, kcache, bt, req, lengths, max_len, got, ws)
     assert torch.equal(got, ref)
+
 
 @pytest.mark.parametrize("T", [3, 1027])
 def test_topk_of_zero_max_len(dev, T):

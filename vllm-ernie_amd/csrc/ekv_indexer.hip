@@ -843,9 +843,11 @@ __global__ void zero_u32_kernel(uint32_t* p, int64_t n) {
 //
 // filter_kernel streams a row's pages for that row alone; a chunk's rows all
 // read the same pages.  Here a workgroup takes kRowsWg consecutive rows, two a
-// wave, and a run of pages, and when the rows are one request's (else each wave
-// streams its rows by itself) every page is loaded once into LDS for all of
-// them.  What is left is VALU work, about 165 instructions per page and row:
+// wave, and a run of pages, and when the rows are one request's every page is
+// loaded once into LDS for all of them; else each wave streams its rows by
+// itself, a page once for both when they are one request's (515 requests of two
+// draft rows at 16K..32K: 0.54 ms in filter_kernel, 0.73 a row after the other, 0.44 here; the
+// whole top-k 1.03, 1.09, 0.80).  What is left is VALU work, about 165 instructions per page and row:
 // relu and the weighted sum are 128 of them, the sums over the lane groups 6
 // (lane swaps that also put token l into lane l), the bounds the rest.  No
 // histogram: the bounds kernel reads the stored bounds.
@@ -968,17 +970,28 @@ filter_rows_kernel(FilterArgs a, uint32_t* bounds) {
     if (s < n[r]) bounds[static_cast<int64_t>(t0 + kRowsWave * wave + r) * a.max_len + s] = wd;
   };
 
-  if (!same) {  // each wave its rows' pages
-#pragma unroll 1
-    for (int r = 0; r < kRowsWave; ++r) {
-      if (n[r] == 0) continue;
-      const PageSource<false> src(a, a.req_ids[t0 + kRowsWave * wave + r], p_end);
-      const int last = min(p_end, (n[r] + kPageTokens - 1) / kPageTokens);
-      for (int lp = p_begin; lp < last; ++lp) {
-        const int64_t page = src.page_of(lp);
-        uint4 kb[4][2];
-        uint32_t ks;
-        src.load(page, kb, ks);
+  if (!same) {
+    // Each wave its rows' pages: two rows of a request (draft rows) share a
+    // page's loads, others go through their pages in step, so that every wave
+    // of the group is at about the same page and finds it in the L2 when
+    // another has read it.
+    const int t = t0 + kRowsWave * wave;
+    const int last[kRowsWave] = {min(p_end, (n[0] + kPageTokens - 1) / kPageTokens),
+                                 min(p_end, (n[1] + kPageTokens - 1) / kPageTokens)};
+    const int32_t req[kRowsWave] = {a.req_ids[min(t, a.rows - 1)], a.req_ids[min(t + 1, a.rows - 1)]};
+    const PageSource<false> src[kRowsWave] = {{a, req[0], p_end}, {a, req[1], p_end}};
+    const bool pair = req[0] == req[1];
+    for (int lp = p_begin; lp < max(last[0], last[1]); ++lp) {
+      uint4 kb[4][2];
+      uint32_t ks;
+      int64_t page = -1;
+#pragma unroll
+      for (int r = 0; r < kRowsWave; ++r) {
+        if (r == 0 ? (pair || lp < last[0]) : !pair && lp < last[1]) {
+          page = src[r].page_of(lp);
+          src[r].load(page, kb, ks);
+        }
+        if (lp >= last[r]) continue;
         float acc[4];
 #pragma unroll
         for (int b = 0; b < 4; ++b) {
@@ -986,12 +999,9 @@ filter_rows_kernel(FilterArgs a, uint32_t* bounds) {
                                  static_cast<int>(kb[b][0].z), static_cast<int>(kb[b][0].w),
                                  static_cast<int>(kb[b][1].x), static_cast<int>(kb[b][1].y),
                                  static_cast<int>(kb[b][1].z), static_cast<int>(kb[b][1].w)};
-          if (r == 0) row_block(op, 0, kv, acc[b]);
-          else row_block(op, 1, kv, acc[b]);
+          row_block(op, r, kv, acc[b]);
         }
-        const float scale = page >= 0 ? __uint_as_float(ks) : 0.0f;
-        if (r == 0) store(0, lp, word(0, acc, scale));
-        else store(1, lp, word(1, acc, scale));
+        store(r, lp, word(r, acc, page >= 0 ? __uint_as_float(ks) : 0.0f));
       }
     }
     return;
