@@ -2818,13 +2818,12 @@ struct SelectArgs {
   const int32_t* cand_idx;
   const int32_t* cand_count; // [T, chunks]
   int32_t chunks;
-  uint32_t* stage_key;       // chunk mode spill: [T, max_len]
+  uint32_t* stage_key;       // chunk mode spill: [T, max_len] keys (kMarked), scores
   int32_t* stage_idx;
   int32_t* out;              // [T, out_stride]
   int64_t out_stride;
   int32_t k;
   int32_t max_len;
-  int32_t sure;              // chunk mode: listed tokens may carry kSureMark
   int32_t seg_groups;        // chunk mode: 0 = lists of kChunk-token chunks, else of
                              // filter_verify_kernel segments (`seg_groups` per row)
   // Optional merged output (merge_swa_topk of the result): [T, merged_stride]
@@ -2857,6 +2856,8 @@ struct SelectSmem {
   uint32_t pmin, pmax;  // range of the current pass's keys
 };
 
+// kMarked (chunk mode): listed tokens may carry kSureMark.
+template <bool kMarked>
 __global__ void __launch_bounds__(kSelThreads) topk_select_kernel(SelectArgs a) {
   extern __shared__ __align__(16) uint8_t smem_raw[];
   SelectSmem& sm = *reinterpret_cast<SelectSmem*>(smem_raw);
@@ -2921,16 +2922,16 @@ __global__ void __launch_bounds__(kSelThreads) topk_select_kernel(SelectArgs a) 
 
   // gather the elements; lo / hi track the range of the keys put in LDS
   uint32_t lo = 0xffffffffu, hi = 0u;
-  // The key of marked tokens (0: none): they are above the threshold and take no
-  // part in the passes that look for it.  No scored token has it (a NaN that
-  // would is taken one lower).  Fewer than k tokens are marked: each has fewer
-  // than k tokens whose upper bound reaches its lower bound.
-  const uint32_t sure_key = a.sure ? 0xffffffffu : 0u;
+  // The key of marked tokens: they are above the threshold and take no part in
+  // the passes that look for it.  No scored token has it (a NaN that would is
+  // taken one lower).  Fewer than k tokens are marked: each has fewer than k
+  // tokens whose upper bound reaches its lower bound.
+  constexpr uint32_t kSureKey = 0xffffffffu;
   int sure = 0;  // this thread's
   int n;
-  const float* gsc = nullptr;      // implicit mode: global scores
-  const uint32_t* gkey = nullptr;  // spilled lists: global keys and indices
-  const int32_t* gidx = nullptr;
+  const float* gsc = nullptr;      // global scores: implicit mode, spilled lists
+  const uint32_t* gkey = nullptr;  // kMarked: global keys of spilled lists
+  const int32_t* gidx = nullptr;   // global indices (spilled lists); null = implicit
   bool in_lds;
   if (a.cand_count == nullptr) {
     n = max(0, min(a.lengths[t], a.max_len));
@@ -3000,10 +3001,9 @@ __global__ void __launch_bounds__(kSelThreads) topk_select_kernel(SelectArgs a) 
         if (p >= n) continue;
         uint32_t key = score_key(sv[q] + 0.0f);
         int32_t ix = iv[q];
-        bool marked = false;
-        if (sure_key != 0u) {
-          marked = ix < 0;
-          key = marked ? sure_key : min(key, sure_key - 1u);
+        const bool marked = kMarked && ix < 0;
+        if constexpr (kMarked) {
+          key = marked ? kSureKey : min(key, kSureKey - 1u);
           ix = static_cast<int32_t>(static_cast<uint32_t>(ix) & ~kSureMark);
         }
         if (marked) ++sure;
@@ -3015,7 +3015,7 @@ __global__ void __launch_bounds__(kSelThreads) topk_select_kernel(SelectArgs a) 
           s_key[p] = key;
           s_idx[p] = ix;
         } else {
-          st_key[p] = key;
+          st_key[p] = kMarked ? key : __float_as_uint(sv[q]);
           st_ix[p] = ix;
         }
       }
@@ -3023,28 +3023,30 @@ __global__ void __launch_bounds__(kSelThreads) topk_select_kernel(SelectArgs a) 
     if (!in_lds) {
       __threadfence_block();
       gkey = st_key;
+      gsc = reinterpret_cast<const float*>(st_key);
       gidx = st_ix;
     }
   }
   for (int off = 32; off > 0; off >>= 1) {
     lo = min(lo, static_cast<uint32_t>(__shfl_xor(static_cast<int>(lo), off)));
     hi = max(hi, static_cast<uint32_t>(__shfl_xor(static_cast<int>(hi), off)));
-    sure += __shfl_xor(sure, off);
+    if constexpr (kMarked) sure += __shfl_xor(sure, off);
   }
   if ((tid & 63) == 0) {
     sm.wmin[tid >> 6] = lo;
     sm.wmax[tid >> 6] = hi;
-    sm.wave[tid >> 6] = sure;
+    if constexpr (kMarked) sm.wave[tid >> 6] = sure;
   }
   __syncthreads();
-  if (sure_key != 0u) {
+  if constexpr (kMarked) {
     sure = 0;
 #pragma unroll
     for (int w = 0; w < kSelThreads / 64; ++w) sure += sm.wave[w];
     __syncthreads();
   }
   auto key_at = [&](int i) -> uint32_t {
-    return in_lds ? s_key[i] : (gkey ? gkey[i] : score_key(gsc[i] + 0.0f));
+    if constexpr (kMarked) return in_lds ? s_key[i] : gkey[i];
+    else return in_lds ? s_key[i] : score_key(gsc[i] + 0.0f);
   };
   auto idx_at = [&](int i) -> int32_t { return in_lds ? s_idx[i] : (gidx ? gidx[i] : i); };
 
@@ -3088,7 +3090,7 @@ __global__ void __launch_bounds__(kSelThreads) topk_select_kernel(SelectArgs a) 
           int bin = -1;
           if (i < n) {
             const uint32_t key = key_at(i);
-            if ((key & mask) == prefix && (sure_key == 0u || key != sure_key)) {
+            if ((key & mask) == prefix && (!kMarked || key != kSureKey)) {
               bin = static_cast<int>((key >> sh) & static_cast<uint32_t>(nb - 1));
               plo = min(plo, key);
               phi = max(phi, key);
@@ -3138,7 +3140,7 @@ __global__ void __launch_bounds__(kSelThreads) topk_select_kernel(SelectArgs a) 
             bool hit = false;
             if (i < n) {
               key = key_at(i);
-              hit = (key & mask) == prefix && (sure_key == 0u || key != sure_key);
+              hit = (key & mask) == prefix && (!kMarked || key != kSureKey);
             }
             const uint64_t bal = __ballot(hit);
             if (bal != 0) {  // wave-uniform
@@ -3240,11 +3242,12 @@ using namespace ekv;
 
 namespace {
 
-void launch_select(const SelectArgs& a, int32_t rows, hipStream_t s) {
+// marked: the lists may carry kSureMark (the many-row path's).
+void launch_select(const SelectArgs& a, int32_t rows, bool marked, hipStream_t s) {
   const int smem = static_cast<int>(sizeof(SelectSmem));
-  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(topk_select_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                      smem);
-  hipLaunchKernelGGL(topk_select_kernel, dim3(rows), dim3(kSelThreads), smem, s, a);
+  const auto kernel = marked ? topk_select_kernel<true> : topk_select_kernel<false>;
+  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+  hipLaunchKernelGGL(kernel, dim3(rows), dim3(kSelThreads), smem, s, a);
 }
 
 int num_chunks(int32_t max_len) { return max_len > 0 ? (max_len + kChunk - 1) / kChunk : 1; }
@@ -3262,7 +3265,7 @@ int64_t count_slots(int64_t T, int32_t max_len) { return T * num_chunks(max_len)
 // workspace: timeouts u32 [4] (cumulative), padded to 256 B | fused-path
 //            counters u32 [kCounterRows, kCounterRow] (kept zero between
 //            calls) | upper u16 [T,L] (4 B per entry reserved) |
-//            cand_score f32 [T,L] | cand_idx i32 [T,L] | stage_key u32 [T,L] |
+//            cand_score f32 [T,L] | cand_idx i32 [T,L] | stage_key 4 B [T,L] |
 //            stage_idx i32 [T,L] | hist u32 [T,4096] | arrive u32 [T] |
 //            kbound u32 [T] (the unfused path's, cleared per call) |
 //            counts i32 [count_slots]
@@ -3467,8 +3470,8 @@ extern "C" int ekv_topk_select(const float* scores, int64_t scores_stride, const
   EKV_CHECK(out_stride >= k, "out_stride must be >= k");
   EKV_CHECK(max_len >= 0 && scores_stride >= max_len, "scores_stride must be >= max_len");
   SelectArgs s{scores, scores_stride, lengths, nullptr, nullptr, nullptr, 0, nullptr, nullptr, out, out_stride, k,
-               max_len, 0, 0, nullptr, 0, 0, nullptr, 0, nullptr, 0, nullptr, 0};
-  launch_select(s, num_tokens, static_cast<hipStream_t>(stream));
+               max_len, 0, nullptr, 0, 0, nullptr, 0, nullptr, 0, nullptr, 0};
+  launch_select(s, num_tokens, false, static_cast<hipStream_t>(stream));
   return ekv_launch_status();
 }
 
@@ -3610,9 +3613,9 @@ int run_select(const TopkQuery& q, const uint8_t* kcache, int64_t page_stride, i
   }
   SelectArgs sel{nullptr, 0, lengths, ws.cand_score, ws.cand_idx, ws.counts, plan.fused ? plan.groups : chunks,
                  ws.stage_key, ws.stage_idx, topk_out, out_stride, k, max_len,
-                 plan.rows ? 1 : 0, plan.fused ? plan.groups : 0, merged_out, merged_stride, merged_width, positions, window,
+                 plan.fused ? plan.groups : 0, merged_out, merged_stride, merged_width, positions, window,
                  merged_slots ? block_table : nullptr, bt_stride, req_ids, num_pages};
-  launch_select(sel, num_tokens, s);
+  launch_select(sel, num_tokens, plan.rows && max_len > 0, s);
   return ekv_launch_status();
 }
 
