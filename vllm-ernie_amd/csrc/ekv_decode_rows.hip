@@ -11,9 +11,9 @@
 //     through LDS, wave w taking rows [8 w, +8);
 //   * weights: exp2(score - reference), row scale folded in, as a pair of bf16
 //     B operands hi = bf16(P), lo = bf16(P - hi), published in LDS.  A head's
-//     reference is its maximum over the steps before, moved when a later step
-//     exceeds it by more than 8 log2 units; a step that exceeds it by more than
-//     100 has its weights computed again, so no barrier waits for the maximum;
+//     reference is its maximum over the steps before; a step that exceeds it by
+//     more than 8 log2 units (rare after the first steps) moves it and has its
+//     weights computed again, so no barrier waits for the maximum and P <= 2^8;
 //   * O^T[128 w, +128) += V^T P^T (the same MFMA).
 // Two barriers a step; the row loads of the two steps after it are in flight.
 // What bounds it: issue (a SIMD issues a conversion or similar VALU
@@ -46,7 +46,6 @@ constexpr int kWaves = 4;
 constexpr int kThreads = 64 * kWaves;
 constexpr int kMaxEntries = 2176;     // index entries of a row (2048 + 128)
 constexpr int kTile = 32;             // cache rows of a step
-constexpr float kRedoSlack = 100.0f;  // log2 units over the reference that have a step's weights computed again (P <= 2**100)
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
@@ -365,8 +364,6 @@ sparse_decode_rows_kernel(DecodeArgs a) {
     for (int i = 0; i < 16; ++i) o[c][i] = 0.0f;
   float mref = -INFINITY;  // the head's reference (log2 units), the same in every wave
   float lsum = 0.0f;       // this lane's share of the head's l
-  float alpha = 1.0f;      // factor that O takes before the next step's products
-  bool rescale = false;    // (wave-uniform) some alpha is not 1
   const float sc2 = a.scale * kLog2e;
   // The head's maximum over a step's rows.
   auto step_max = [&]() -> float {
@@ -512,30 +509,15 @@ sparse_decode_rows_kernel(DecodeArgs a) {
       for (int j = 0; j < SM::kLoadsPerWave; ++j) ro[j] = sm.roff[tl.row[j]];
     }
     const float mx = step_max();
-    float f = alpha;
-    bool scale = rescale;
-    alpha = 1.0f;
-    rescale = false;
     if (__any(mx > mref + kRescaleSlack)) {  // the same in every wave (also a first finite maximum)
-      if (__any(mx > mref + kRedoSlack)) {
-        const float al = move_ref(mx);
-        f *= al;
-        scale = true;
-        lsum *= al;
-        weights();
-        __syncthreads();
-        read_p();
-        lsum += psum;
-      } else {
-        lsum += psum;
-        alpha = move_ref(mx);
-        rescale = true;
-        lsum *= alpha;
-      }
-    } else {
-      lsum += psum;
+      const float al = move_ref(mx);
+      scale_o(al);
+      lsum *= al;
+      weights();
+      __syncthreads();
+      read_p();
     }
-    if (scale) scale_o(f);
+    lsum += psum;
 #pragma unroll
     for (int c = 0; c < 4; ++c) raw[kRaw - 1][c] = pv_read<D, BF16>(img, kRaw - 1, wave, c);
     if (!BF16 && s + 1 < ntiles) read_k(s + 1);
@@ -564,7 +546,6 @@ sparse_decode_rows_kernel(DecodeArgs a) {
       }
     }
   }
-  if (rescale) scale_o(alpha);
 
   // Epilogue: the waves' sums of weights meet, wave 0 finishes the heads'
   // softmax (the sink, the lse) and publishes the output factors.
