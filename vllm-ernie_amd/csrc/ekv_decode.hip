@@ -678,11 +678,13 @@ sparse_decode_kernel(DecodeArgs a) {
 // Wave w of a head sums splits w, w + kW, ...; with kW = 4 the four sums meet
 // in LDS, each thread finishing two channels.  Bound by memory latency (the
 // partials, 2 KB per split and head, come from other XCDs' writes), so the
-// splits' loads go out together.  Many splits a row: 4 waves (one row of 68
-// splits: 6.7 us, 14.7 with a wave per head).  Up to 16: a wave per head (32
-// rows of 8: 8.4 us, 10.4 with 4 waves; 64 of 4: 7.6, 12.7; 27 of 9: the same
-// with the partials in the caches, but a step on a workspace just allocated
-// 431 us against 481-519).  Rows finished by their only split are skipped.
+// splits' loads go out together.  With kW = 1 there is a workgroup per 4 heads
+// and row; while these are fewer than half the CUs, 4 waves a head: decode and
+// combine of 1, 4, 7 rows of 2176 entries at 64 heads 30.4, 32.0, 31.4 us with
+// a wave per head, 22.2, 28.1, 29.4 with 4; 8, 12, 16, 32 rows 29.9, 29.0, 30.4, 37.8
+// and 32.4, 28.9, 30.7, 39.2.  At 32 heads 8, 15, 16 rows 27.7, 27.3, 26.4 and
+// 24.8, 24.8, 25.4, at 16 heads 8, 25, 32 rows 22.1, 25.7, 27.8 and 19.5, 24.5,
+// 28.0.  Rows finished by their only split are skipped.
 template <int kW>
 __global__ void __launch_bounds__(256) decode_combine_kernel(
     const float* ws_o, const float* ws_ml, const int2* ws_rows, int32_t heads, const float* sinks,
@@ -862,7 +864,7 @@ extern "C" int ekv_sparse_mla_decode(const uint16_t* q, int64_t q_tok_stride, in
   }
   int rc = ekv_launch_status();
   if (rc) return rc;
-  if (groups > 16 * static_cast<int64_t>(num_tokens))  // more than 16 splits a row
+  if (heads * static_cast<int64_t>(num_tokens) < 512)
     hipLaunchKernelGGL(decode_combine_kernel<4>, dim3(heads, num_tokens), dim3(256), 0, s, ws_o, ws_ml, ws_rows, heads,
                        sinks, out, out_tok_stride, out_head_stride, lse, lse_stride);
   else
