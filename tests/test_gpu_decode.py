@@ -247,3 +247,60 @@ def test_decode_hca_shapes_vs_oracle(dev, case):
     ref_o, ref_l = od.sparse_mla_decode(q, lambda s: od.gather_rows_fp8(pool_np, s, dim), idx, 256 ** -0.5, 512,
                                         sinks, lens)
     _check(out, lse, ref_o, ref_l, H)
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("dim,heads,T,width", [(512, 64, 5, 385), (512, 16, 5, 900), (512, 64, 20, 1153),
+                                               (512, 16, 40, 385), (576, 48, 9, 500), (576, 16, 5, 2176)])
+def test_few_row_kernel_edges(dev, bf16, dim, heads, T, width):
+    """Few long rows, split over workgroups and combined (by four waves a head
+    and by one), with lengths at the edges of its 32-entry tiles."""
+    from ernie_kv import ops
+
+    rng = np.random.default_rng(dim + heads + T + width)
+    pages = 40
+    if bf16:
+        rows = randn_bf16(rng, (pages * 64, dim))
+        cache, fetch = bf16_tensor(rows, dev).view(-1, 64, dim), lambda s: od.gather_rows_bf16(rows, s)
+    else:
+        pool = _fp8_pool(rng, pages, dim)
+        cache, fetch = to_dev(pool, dev), lambda s: od.gather_rows_fp8(pool, s, dim)
+    idx = rng.integers(-200, pages * 64, (T, width)).astype(np.int32)
+    idx = np.maximum(idx, -1)
+    lengths = rng.integers(0, width + 1, T).astype(np.int32)
+    lengths[:5] = [0, 1, 31, 33, width]
+    q = randn_bf16(rng, (T, heads, dim))
+    sinks = rng.standard_normal(heads).astype(np.float32)
+    out = torch.zeros((T, heads, 512), dtype=torch.bfloat16, device=dev)
+    lse = torch.zeros((T, heads), dtype=torch.float32, device=dev)
+    ops.sparse_mla_decode(bf16_tensor(q, dev), cache, to_dev(idx, dev), 256 ** -0.5, out, lse,
+                          sinks=to_dev(sinks, dev), lengths=to_dev(lengths, dev), cache_bf16=bf16)
+    ref_o, ref_l = od.sparse_mla_decode(q, fetch, idx, 256 ** -0.5, 512, sinks, lengths)
+    _check(out, lse, ref_o, ref_l, heads)
+
+
+def test_decode_cancelling_pair_padded(dev):
+    """test_decode_cancelling_pair in rows padded to a width of the few-row kernel."""
+    from ernie_kv import ops
+
+    rng = np.random.default_rng(6)
+    dim, H, T, width = 576, 64, 16, 420
+    v = randn_bf16(rng, (1, dim), 2.0)
+    rows = np.concatenate([v, -v, np.zeros((62, dim), np.float32)])
+    pool = np.zeros((1, paged.fp8_page_bytes(dim)), np.uint8)
+    c, sc = quantize_rows(rows)
+    paged.write_fp8_rows(pool, np.arange(64), c, sc, dim)
+    k0 = od.gather_rows_fp8(pool, np.array([0]), dim)[0]
+    q = np.zeros((T, H, dim), np.float32)
+    for t in range(T):
+        target = 10.0 ** rng.uniform(-4, -2) * 16.0 / 2.0
+        q[t] = (k0 * target / float(k0 @ k0))[None, :]
+    q = bf16_round_np(q)
+    idx = np.full((T, width), -1, np.int32)
+    idx[:, 3], idx[:, 20] = 0, 1
+    out = torch.zeros((T, H, 512), dtype=torch.bfloat16, device=dev)
+    lse = torch.zeros((T, H), dtype=torch.float32, device=dev)
+    ops.sparse_mla_decode(bf16_tensor(q, dev), to_dev(pool, dev), to_dev(idx, dev), 256 ** -0.5, out, lse)
+    ref_o, ref_l = od.sparse_mla_decode(q, lambda s: od.gather_rows_fp8(pool, s, dim), idx, 256 ** -0.5, 512)
+    assert np.abs(ref_o).max() < 0.05 * np.abs(k0).max()  # the two terms nearly cancel
+    _check(out, lse, ref_o, ref_l, H)

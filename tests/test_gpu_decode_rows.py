@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import bf16_tensor, bf16_values, randn_bf16, to_dev
+from helpers import bf16_tensor, permuted_block_table, randn_bf16, to_dev
 from oracle import decode as od
 from oracle import paged
 from test_gpu_decode import _check, _fp8_pool
@@ -72,6 +72,36 @@ def test_dispatch_lines(dev, T, heads, width, dim, bf16):
     lengths = rng.integers(0, 40, T).astype(np.int32)
     lengths[::50] = width
     _run(dev, rng, dim, heads, np.maximum(idx, -1), lengths, bf16)
+
+
+@pytest.mark.parametrize("T,width,bf16", [(5, 200, False), (193, 300, False), (9, 100, True)])
+def test_rows_block_table(dev, T, width, bf16):
+    """Request-local indices through the block table: unmapped pages, pages and
+    entries past the table."""
+    from ernie_kv import ops
+
+    rng = np.random.default_rng(T)
+    B, P, dim, H = 3, 12, 576, 64
+    bt = permuted_block_table(rng, B, P)
+    bt[1, 3], bt[2, 5] = -1, B * P + 4
+    req = rng.integers(0, B, T).astype(np.int32)
+    logical = np.maximum(rng.integers(-100, (P + 2) * 64, (T, width)), -1).astype(np.int32)
+    lengths = rng.integers(0, width + 1, T).astype(np.int32)
+    if bf16:
+        rows = randn_bf16(rng, (B * P * 64, dim))
+        cache, fetch = bf16_tensor(rows, dev).view(-1, 64, dim), lambda s: od.gather_rows_bf16(rows, s)
+    else:
+        pool = _fp8_pool(rng, B * P, dim)
+        cache, fetch = to_dev(pool, dev), lambda s: od.gather_rows_fp8(pool, s, dim)
+    q = randn_bf16(rng, (T, H, dim))
+    out = torch.zeros((T, H, 512), dtype=torch.bfloat16, device=dev)
+    lse = torch.zeros((T, H), dtype=torch.float32, device=dev)
+    ops.sparse_mla_decode(bf16_tensor(q, dev), cache, to_dev(logical, dev), 256 ** -0.5, out, lse, cache_bf16=bf16,
+                          lengths=to_dev(lengths, dev), block_table=to_dev(bt, dev), req_ids=to_dev(req, dev))
+    page = np.where((logical >= 0) & (logical < P * 64), bt[req[:, None], np.clip(logical, 0, P * 64 - 1) // 64], -1)
+    glob = np.where((page >= 0) & (page < B * P), page * 64 + logical % 64, -1)
+    ref_o, ref_l = od.sparse_mla_decode(q, fetch, glob, 256 ** -0.5, 512, None, lengths)
+    _check(out, lse, ref_o, ref_l, H)
 
 
 @pytest.mark.parametrize("factor", [8.0, 96.0])

@@ -30,6 +30,8 @@ def _case(dev, T, n_seqs, order, max_len, kind, seed):
         k = k[torch.randint(0, 30, (n,), device=dev, generator=g)]
     elif kind == "constant":
         k = k[:1].expand(n, 128)
+    elif kind == "peaks":  # most keys tied, some above and below
+        k = torch.where((torch.arange(n, device=dev) % 400 == 7)[:, None], k, k[:1])
     elif kind == "overflow":  # of every 7 keys one scores beyond fp32 (about half of them +inf, half -inf)
         k[::7] *= 1e37
     elif kind == "all inf":
@@ -38,6 +40,8 @@ def _case(dev, T, n_seqs, order, max_len, kind, seed):
     if kind == "unmapped":
         bt[:, 1] = -1
         bt[-1, -1] = n_seqs * pages + 7
+    elif kind == "holes":
+        bt[:, 5::9] = -1
     if kind == "nan":
         kcache[:, 64 * 128:].view(torch.float32)[:, ::9] = float("nan")
     if order.isdigit():  # that many draft rows a request
@@ -45,7 +49,8 @@ def _case(dev, T, n_seqs, order, max_len, kind, seed):
     else:
         req = np.sort(rng.integers(0, n_seqs, T)) if order == "runs" else rng.integers(0, n_seqs, T)
     req = req.astype(np.int32)
-    lengths = np.minimum(max_len, 1 + np.arange(T) % (max_len + 40)).astype(np.int32)
+    step = 7919 if max_len > 4 * T else 1  # (rows of all lengths)
+    lengths = np.minimum(max_len, 1 + step * np.arange(T) % (max_len + 40)).astype(np.int32)
     q = torch.randn(T, 64, 128, device=dev, generator=g).bfloat16()
     w = torch.randn(T, 64, device=dev, generator=g).bfloat16()
     if kind in ("overflow", "all inf"):
@@ -67,11 +72,16 @@ def _case(dev, T, n_seqs, order, max_len, kind, seed):
     (1026, 3, "mixed", 600, 100, "nan"),
     (1030, 515, "2", 700, 100, "unmapped"),
     (1027, 343, "3", 400, 64, "ties"),
+    (2100, 1, "runs", 50_000, 256, "holes"),  # runs of 66 pages, several 8192-token groups a row
+    (1030, 1, "runs", 40_003, 256, "peaks"),  # more candidates than the select's LDS holds, some of them sure
+    (300, 2, "runs", 60_000, 2048, "normal"),
+    (260, 130, "2", 50_000, 512, "ties"),
 ])
 def test_many_rows_topk_matches_exact_scores(dev, T, n_seqs, order, max_len, k, kind):
     from ernie_kv import ops
 
     q8, w, dig, kcache, bt, req, lengths = _case(dev, T, n_seqs, order, max_len, kind, T + max_len)
+    assert not ops.dsa_decode_prologue_folds(T, max_len)  # (the one-launch top-k does not take it)
     scores = torch.full((T, max_len), float("nan"), device=dev)
     ops.indexer_score(dig, w, kcache, bt, req, lengths, max_len, scores)
     n_inf = int((scores == float("inf")).sum(1).max())
@@ -118,3 +128,28 @@ def test_topk_of_zero_max_len(dev, T):
         else:
             ops.indexer_topk(q8, dig, w, kcache, bt, req, lengths, 0, got, ws)
         assert (got == -1).all()
+
+
+@pytest.mark.parametrize("slots", [False, True])
+def test_many_rows_merged_output(dev, slots):
+    """The top-k merged with the window, as token indices and as cache slots."""
+    from ernie_kv import ops
+
+    T, max_len, k, window = 1027, 900, 128, 64
+    q8, w, dig, kcache, bt, req, lengths = _case(dev, T, 3, "runs", max_len, "unmapped", 9)
+    positions = lengths.long() + window - 1  # the rows' keys end where their windows begin
+    ws = ops.indexer_topk_workspace(T, max_len, dev)
+    topk, got = (torch.empty((T, k + d), dtype=torch.int32, device=dev) for d in (0, window))
+    ops.indexer_topk_merged(q8, dig, w, kcache, bt, req, lengths, max_len, topk, ws, merged=got, positions=positions,
+                            window=window, merged_slots=slots)
+    plain = torch.empty((T, k), dtype=torch.int32, device=dev)
+    ops.indexer_topk(q8, dig, w, kcache, bt, req, lengths, max_len, plain)
+    assert torch.equal(topk, plain)
+    ref = torch.empty_like(got)
+    ops.merge_swa_topk(plain, ref, positions, window)
+    if slots:
+        i = ref.long()
+        page = torch.where((i >= 0) & (i // 64 < bt.shape[1]),
+                           bt[req.long()[:, None], (i // 64).clamp(0, bt.shape[1] - 1)].long(), -1)
+        ref = torch.where((page >= 0) & (page < kcache.shape[0]), page * 64 + i % 64, -1).int()
+    assert torch.equal(got, ref)

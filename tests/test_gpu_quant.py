@@ -87,3 +87,49 @@ def test_vha_inv_rope_fp8_quant(dev, num_tokens):
     aligned = (num_tokens + 3) // 4 * 4
     full = torch.empty(0, dtype=torch.int32, device=dev).set_(got.scale.untyped_storage()).view(groups, hpg, aligned)
     assert (full[..., num_tokens:] == 0).all()
+
+
+def test_sigmoid_every_finite_gate(dev):
+    """The gate's bf16 sigmoid is that of the fp64 evaluation for every finite
+    bf16 gate: four neighbouring gates share a group, each times 32 consecutive
+    bf16 values, so that a sigmoid one bf16 step off changes some code."""
+    from ernie_kv import attention as A
+
+    bits = np.arange(1 << 16, dtype=np.uint32)
+    bits = bits[(bits & 0x7F80) != 0x7F80]
+    g = np.repeat(bits << 16, 32).view(np.float32)
+    x = np.tile((1 + np.arange(32) / 128).astype(np.float32), len(bits))
+    g, x = g.reshape(-1, 8192), x.reshape(-1, 8192)
+    q, s = A.sigmoid_mul_quant_fp8(bf16_tensor(x, dev), bf16_tensor(g, dev))
+    codes, packed = oq.sigmoid_mul_quant(x, g)
+    assert np.array_equal(q.view(torch.uint8).cpu().numpy(), codes)
+    assert np.array_equal(s.cpu().numpy(), packed)
+
+
+@pytest.mark.parametrize("num_tokens", [513, 769, 1030])
+def test_vha_tokens_of_one_workgroup(dev, num_tokens):
+    """Workgroups that walk over three and more tokens, the last round ragged:
+    the bytes of calls of at most 200 tokens (one a workgroup), and the same
+    bytes in an output that is not 16-byte aligned."""
+    from ernie_kv import _lib, ops
+
+    g = torch.Generator(device=dev).manual_seed(num_tokens)
+    rnd = lambda *s: torch.randn(*s, device=dev, generator=g)  # noqa: E731
+    o, mix = rnd(num_tokens, 64, 512).bfloat16(), (torch.eye(64, device=dev) + rnd(64, 64) / 16).bfloat16()
+    positions = torch.randint(0, 4096, (num_tokens,), device=dev, generator=g)
+    cs = to_dev(oi.rope_cos_sin(np.arange(4096), 64, 1e4), dev)
+    data, scale = ops.vha_inv_rope_fp8_quant(o, mix, positions, cs, 8, 448, 64)
+    for a in range(0, num_tokens, 200):
+        d, s = ops.vha_inv_rope_fp8_quant(o[a:a + 200], mix, positions[a:a + 200], cs, 8, 448, 64)
+        assert torch.equal(data[a:a + 200].view(torch.uint8), d.view(torch.uint8)) and torch.equal(scale[a:a + 200], s)
+    n, aligned = data.numel(), ops.tma_aligned_rows(num_tokens)
+    raw = torch.zeros(n + 64, dtype=torch.uint8, device=dev)
+    at = raw[4:4 + n]
+    assert at.data_ptr() % 16 == 4
+    scale4 = torch.empty((8, 8, aligned), dtype=torch.int32, device=dev)
+    _lib.call("ekv_vha_inv_rope_fp8_quant", o.data_ptr(), o.stride(0), o.stride(1), num_tokens, 64, mix.data_ptr(),
+              positions.data_ptr(), cs.data_ptr(), cs.stride(0), 8, 448, 64, at.data_ptr(), scale4.data_ptr(), aligned,
+              ops._stream())
+    assert torch.equal(at.view(8, num_tokens, 4096), data.transpose(0, 1).view(torch.uint8))
+    assert torch.equal(scale4.permute(2, 0, 1)[:num_tokens], scale)
+    assert (raw[:4] == 0).all() and (raw[4 + n:] == 0).all()
