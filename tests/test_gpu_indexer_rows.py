@@ -40,7 +40,7 @@ def _case(dev, T, n_seqs, order, max_len, kind, seed):
     if kind == "unmapped":
         bt[:, 1] = -1
         bt[-1, -1] = n_seqs * pages + 7
-    elif kind == "holes":
+    elif kind in ("holes", "at most 0"):
         bt[:, 5::9] = -1
     if kind == "nan":
         kcache[:, 64 * 128:].view(torch.float32)[:, ::9] = float("nan")
@@ -57,6 +57,8 @@ def _case(dev, T, n_seqs, order, max_len, kind, seed):
         w = w * 1024
     if kind == "all inf":
         q, w = q.abs(), w.abs()
+    elif kind == "at most 0":  # the unmapped pages' scores of 0 are the largest
+        w = -w.abs()
     return (*ops.indexer_q_quant(q, w), kcache, to_dev(bt, dev), to_dev(req, dev), to_dev(lengths, dev))
 
 
@@ -76,6 +78,9 @@ def _case(dev, T, n_seqs, order, max_len, kind, seed):
     (1030, 1, "runs", 40_003, 256, "peaks"),  # more candidates than the select's LDS holds, some of them sure
     (300, 2, "runs", 60_000, 2048, "normal"),
     (260, 130, "2", 50_000, 512, "ties"),
+    (1030, 2, "runs", 500, 40, "at most 0"),
+    (1030, 2, "mixed", 500, 64, "at most 0"),
+    (1030, 2, "runs", 500, 90, "at most 0"),
 ])
 def test_many_rows_topk_matches_exact_scores(dev, T, n_seqs, order, max_len, k, kind):
     from ernie_kv import ops

@@ -864,11 +864,14 @@ constexpr int kRowsWg = kRowsWave * kRowsWaves;
 constexpr int kRowsBufs = 3;                       // LDS page buffers: one in use, two loading
 constexpr int kRowsPage = kIdxPageBytes + 256;     // values, then the 64 scales
 
-// 16-bit key of a bf16 bound (order of score_key; -0 as +0).
-__device__ __forceinline__ uint32_t bound_key(uint32_t bits) {
-  if (bits == 0x8000u) bits = 0u;
-  return (bits & 0x8000u) ? (~bits & 0xffffu) : (bits | 0x8000u);
+// The 16-bit keys of a token's two bf16 bounds (order of score_key; -0 just
+// below +0), U's in the high half.
+typedef short bound_i16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t bound_keys(uint32_t word) {
+  const bound_i16x2 sign = __builtin_bit_cast(bound_i16x2, word) >> 15;
+  return word ^ (__builtin_bit_cast(uint32_t, sign) | 0x80008000u);
 }
+constexpr uint32_t kPlusZero = 0x8000u, kMinusZero = 0x7fffu;
 
 // Sum over the four lane groups of each of a page's four blocks; lane l gets
 // that of token l = 16 b + col.
@@ -1085,7 +1088,9 @@ filter_rows_kernel(FilterArgs a, uint32_t* bounds) {
 // exact score (by a select of k or more; kfilter[t] keeps k).  A row of at
 // most k tokens has no bounds: every token is a candidate, none vouched for.
 // One workgroup per row: the bounds' high 12 key bits, then the low 4 of the
-// two threshold bins.
+// two threshold bins.  VALU bound (a CU takes a row of 75000 words in about 40
+// us); 1024 threads are faster for fewer rows than CUs take (300 rows of 75000:
+// 71 us, 61) and slower for a chunk (4096 of 24000: 116, 136).
 __global__ void __launch_bounds__(512) row_bounds_kernel(const uint32_t* bounds, const int32_t* lengths,
                                                          int32_t max_len, int32_t k, uint32_t* kbound, uint32_t* kin,
                                                          uint32_t* kfilter) {
@@ -1118,8 +1123,9 @@ __global__ void __launch_bounds__(512) row_bounds_kernel(const uint32_t* bounds,
 #pragma unroll
     for (int j = 0; j < kPer; ++j) {
       if (i0 + 512 * j + tid >= n) break;
-      atomicAdd(&s_hist[0][bound_key(w[j] >> 16) >> 4], 1u);
-      atomicAdd(&s_hist[1][bound_key(w[j] & 0xffffu) >> 4], 1u);
+      const uint32_t kk = bound_keys(w[j]);
+      atomicAdd(&s_hist[0][kk >> 20], 1u);
+      atomicAdd(&s_hist[1][(kk >> 4) & 0xfffu], 1u);
     }
   }
   __syncthreads();
@@ -1159,9 +1165,9 @@ __global__ void __launch_bounds__(512) row_bounds_kernel(const uint32_t* bounds,
 #pragma unroll
     for (int j = 0; j < kPer; ++j) {
       if (i0 + 512 * j + tid >= n) break;
-      const uint32_t ku = bound_key(w[j] >> 16), kl = bound_key(w[j] & 0xffffu);
-      if (static_cast<int>(ku >> 4) == bin[0]) atomicAdd(&s_low[0][ku & 15u], 1u);
-      if (static_cast<int>(kl >> 4) == bin[1]) atomicAdd(&s_low[1][kl & 15u], 1u);
+      const uint32_t kk = bound_keys(w[j]);
+      if (static_cast<int>(kk >> 20) == bin[0]) atomicAdd(&s_low[0][(kk >> 16) & 15u], 1u);
+      if (static_cast<int>((kk >> 4) & 0xfffu) == bin[1]) atomicAdd(&s_low[1][kk & 15u], 1u);
     }
   }
   __syncthreads();
@@ -1173,8 +1179,9 @@ __global__ void __launch_bounds__(512) row_bounds_kernel(const uint32_t* bounds,
       above += c;
     }
     const uint32_t key = static_cast<uint32_t>(bin[tid] * 16 + low);
-    if (tid == 0) kin[t] = key;
-    else kbound[t] = key << 16;
+    // -0 and +0 are one bound: U of -0 reaches a score of +0
+    if (tid == 0) kin[t] = key == kMinusZero ? kPlusZero : key;
+    else kbound[t] = (key == kPlusZero ? kMinusZero : key) << 16;
   }
 }
 
@@ -1291,9 +1298,10 @@ __global__ void __launch_bounds__(256) verify_kernel(VerifyArgs a) {
       uint32_t flags = 0, sure = 0;
 #pragma unroll
       for (int j = 0; j < kPer; ++j) {
-        if (start + j < len && bound_key(wd[cc][j] >> 16) >= kb16) {
+        const uint32_t kk = bound_keys(wd[cc][j]);
+        if (start + j < len && (kk >> 16) >= kb16) {
           flags |= 1u << j;
-          if (bound_key(wd[cc][j] & 0xffffu) > kin) sure |= 1u << j;
+          if ((kk & 0xffffu) > kin) sure |= 1u << j;
         }
       }
       // positions in the chunk's list (all candidates) and in the scored list
