@@ -393,7 +393,8 @@ int64_t ekv_indexer_topk_counter_bytes(void);
  */
 int32_t ekv_indexer_set_spin_limit(int32_t polls);
 
-/* Workspace bytes ekv_sparse_mla_decode needs. */
+/* Workspace bytes ekv_sparse_mla_decode needs (asked of every call, also of
+ * those that take the whole-row kernel, which writes no partials). */
 int64_t ekv_sparse_mla_decode_workspace_size(int32_t num_tokens, int32_t heads, int32_t width);
 
 /*
@@ -467,8 +468,9 @@ int ekv_indexer_filter_dots(const uint8_t* q_codes, const uint8_t* k_codes, int3
  * split partials go to a 64 MiB device array inside the library (one per
  * GPU, held until the process ends); a call needing more
  * (ekv_sparse_mla_decode_workspace_size > 64 MiB, e.g. beyond ~150 query
- * rows of 2176 entries at 64 heads) fails with status 1.  Calls that overlap
- * on one GPU (different streams) race on that array.  Allocates nothing.
+ * rows of 2176 entries at 64 heads) fails with status 1, also where the call
+ * would take the whole-row kernel, which writes no partials.  Calls that
+ * overlap on one GPU (different streams) race on that array.  Allocates nothing.
  */
 int ekv_sparse_mla_decode_noalloc(const uint16_t* q, int64_t q_tok_stride, int64_t q_head_stride,
                                   int32_t num_tokens, int32_t heads, int32_t dim, const uint8_t* cache,

@@ -31,10 +31,11 @@
 // A prologue resolves every index entry to a cache slot (block table lookup)
 // and drops the masked ones (order kept), so a row costs its valid entries.
 // Against splits of 32 tiles with fp32 partials and a combine (the few-row
-// kernel): 4096 rows of 2176 entries 2.93 -> 2.23 ms, 2331 rows of 2176 of
-// which 515 valid on average 1.70 -> 0.43 ms, 6000 rows of about 137 entries
-// 0.75 -> 0.42 ms (64 heads, fp8).  3600 cycles a pair of 32-row steps on a CU
-// (two workgroups), of which the matrix cores work 1600.
+// kernel): 4096 rows of 2176 entries 2.78 -> 2.07 ms, 2331 rows of 2176 of
+// which 515 valid on average 1.63 -> 0.39 ms, 6000 rows of about 137 entries
+// 0.73 -> 0.40 ms (64 heads, fp8).  4096 rows, by the counters: 4000 cycles a
+// pair of 32-row steps on a CU (two workgroups), prologues and epilogues
+// included, of which the matrix cores work 1600 (40%).
 #include "ekv_decode.h"
 #include "ekv_internal.h"
 
@@ -138,7 +139,7 @@ __device__ __forceinline__ int slot_row(int hl, int m) { return m < 4 ? 4 * hl +
 // (64 k + i) / kChunks, stored chunk j = (64 k + i) % kChunks, which holds
 // row chunk swz(j, r).  Rows past the last valid entry load cache row 0
 // (zeroed once the step has landed).  Wave w issues the instructions
-// k = w + 8 j; this lane then copies byte col[j] on of step entry row[j].
+// k = w + 4 j; this lane then copies byte col[j] on of step entry row[j].
 template <int D, bool BF16>
 struct TileLanes {
   static constexpr int kN = DecodeSmem<D, BF16>::kLoadsPerWave;

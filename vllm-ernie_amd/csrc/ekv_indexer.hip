@@ -846,14 +846,17 @@ __global__ void zero_u32_kernel(uint32_t* p, int64_t n) {
 // wave, and a run of pages, and when the rows are one request's every page is
 // loaded once into LDS for all of them; else each wave streams its rows by
 // itself, a page once for both when they are one request's (515 requests of two
-// draft rows at 16K..32K: 0.54 ms in filter_kernel, 0.73 a row after the other, 0.44 here; the
-// whole top-k 1.03, 1.09, 0.80).  What is left is VALU work, about 165 instructions per page and row:
-// relu and the weighted sum are 128 of them, the sums over the lane groups 6
-// (lane swaps that also put token l into lane l), the bounds the rest.  No
-// histogram: the bounds kernel reads the stored bounds.
-// 4096 rows ending at 32768: 2.35 -> 1.01 ms (the bounds kernel adds 0.18; the
-// candidates left to score fall from 3100 to about 1800 a row, verify 1.26 ->
-// 0.99 ms, and the select 0.52 -> 0.31).
+// draft rows at 16K..32K: 0.54 ms in filter_kernel, 0.73 a row after the other,
+// 0.44 here; the whole top-k 1.03, 1.09, 0.80).  What is left is VALU work, 163
+// instructions and 16 MFMAs per page and row (counted): relu and the weighted
+// sum are 128 of them, the sums over the lane groups 6 (lane swaps that also
+// put token l into lane l), the bounds the rest.  No histogram: the bounds
+// kernel reads the stored bounds.
+// 4096 rows ending at 32768: 2.12 -> 0.96 ms (the bounds kernel adds 0.16; the
+// verify takes 1.15 -> 0.79 ms, with at most 1360 tokens a row left to score,
+// and the select 0.51 -> 0.30).  Rows of different requests gain as long as the
+// verify and select save more than the wider words cost: 300 requests of
+// 20K..40K 446 -> 419 us, of 50K..100K 866 -> 911.
 //
 // Each token gets one word: U_s (bf16, rounded up) in the high half, L_s (bf16,
 // rounded down) in the low one.
@@ -1040,9 +1043,9 @@ filter_rows_kernel(FilterArgs a, uint32_t* bounds) {
     return id >= 0;
   };
   // A page's words are stored at the start of the next iteration, ahead of the
-  // loads issued there, so that what follows the loads of page p + 1 is known:
-  // the stores of page p - 1 and the loads of page p + 2, which may stay in
-  // flight when page p is done.
+  // loads issued there, so that only the loads of page p + 2 follow those of
+  // page p + 1: they stay in flight when page p is done (the stores of page
+  // p - 1 have to be through by then).
   uint32_t wd[kRowsWave];
   bool ok0 = load(p_begin), ok1 = p_begin + 1 < p_end ? load(p_begin + 1) : false;
   wait_vm<0>();
@@ -1220,7 +1223,7 @@ constexpr int kVerifyPages = kVerifyChunks * kChunk / kPageTokens;
 
 // kRows: the bounds are filter_rows_kernel's words, and a candidate whose
 // lower bound is above kin is selected in any case: it is listed unscored,
-// its index marked with kSureMark (about two thirds of a row's candidates).
+// its index marked with kSureMark (more than half of a row's candidates).
 template <bool kFp4, bool kRows = false>
 __global__ void __launch_bounds__(256) verify_kernel(VerifyArgs a) {
   __shared__ uint32_t s_table[256];  // fp8: digit table; fp4: q scale words
